@@ -245,40 +245,110 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(LinearArgs a, const
   store_run4(a, a.out, a.ldo, a.epilogue == TF_EPILOGUE_RESIDUAL, row, col, v, true);
 }
 
+// The same under SiLU*mul (N % 8 == 0): four outputs per thread, the runs of their gate and up
+// columns summed one after the other.
+__global__ __launch_bounds__(256) void splitk_reduce4_silu_kernel(LinearArgs a, const float* __restrict__ ws,
+                                                                  int split) {
+  const int half = a.n >> 1;
+  const int64_t total = (int64_t)a.m * a.n;
+  const int64_t o = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (o >= (int64_t)a.m * half) return;
+  const int row = (int)(o / half);
+  const int col = (int)(o - (int64_t)row * half);
+  const float rs = row_scale(a, row);
+  float v[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float* const src = ws + (int64_t)row * a.n + h * half + col;
+    f4 p[kMaxSplitK];
+#pragma unroll
+    for (int s = 0; s < kMaxSplitK; ++s)
+      if (s < split) p[s] = *reinterpret_cast<const f4*>(src + (int64_t)s * total);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float acc = p[0][j];
+#pragma unroll
+      for (int s = 1; s < kMaxSplitK; ++s)
+        if (s < split) acc += p[s][j];
+      acc = acc * rs;
+      if (a.bias) acc += half_bits_to_float(a.bias[h * half + col + j]);
+      v[h][j] = acc;
+    }
+  }
+  uint16_t r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = finish_silu_mul(v[0][j], v[1][j]);
+  *reinterpret_cast<u2*>(a.out + (int64_t)row * a.ldo + col) =
+      u2{(uint32_t)r[0] | ((uint32_t)r[1] << 16), (uint32_t)r[2] | ((uint32_t)r[3] << 16)};
+}
+
 }  // namespace
 
-// SiLU*mul over an fp16 y [m, n] (row stride n) staged in the workspace.
+// SiLU*mul over an fp16 y [m, n] (row stride n) staged in the workspace, V outputs per thread (4
+// where the out rows are in 4-element units: N % 16 == 0, so the halves of a y row are).
+template <int V>
 __global__ void silu_mul_kernel(LinearArgs a, const uint16_t* __restrict__ y) {
   const int half = a.n >> 1;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (i >= (int64_t)a.m * half) return;
   const int64_t row = i / half;
   const int64_t col = i % half;
-  a.out[row * a.ldo + col] =
-      finish_silu_mul(half_bits_to_float(y[row * a.n + col]), half_bits_to_float(y[row * a.n + half + col]));
+  const uint16_t* const gate = y + row * a.n + col;
+  uint16_t* const out = a.out + row * a.ldo + col;
+  if (V == 4) {
+    const u2 g = *reinterpret_cast<const u2*>(gate), u = *reinterpret_cast<const u2*>(gate + half);
+    uint32_t h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      h[j] = finish_silu_mul(half_bits_to_float((uint16_t)(g[j >> 1] >> (16 * (j & 1)))),
+                             half_bits_to_float((uint16_t)(u[j >> 1] >> (16 * (j & 1)))));
+    *reinterpret_cast<u2*>(out) = u2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+  } else {
+    out[0] = finish_silu_mul(half_bits_to_float(gate[0]), half_bits_to_float(gate[half]));
+  }
 }
 
 int silu_mul_staged(const LinearArgs& a, const float* ws, hipStream_t stream) {
   const int64_t total = (int64_t)a.m * (a.n >> 1);
-  silu_mul_kernel<<<(unsigned)cdiv(total, 256), 256, 0, stream>>>(a, reinterpret_cast<const uint16_t*>(ws));
+  const uint16_t* const y = reinterpret_cast<const uint16_t*>(ws);
+  if ((a.ldo & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(ws)) & 7) == 0)
+    silu_mul_kernel<4><<<(unsigned)cdiv(total / 4, 256), 256, 0, stream>>>(a, y);
+  else
+    silu_mul_kernel<1><<<(unsigned)cdiv(total, 256), 256, 0, stream>>>(a, y);
   return check_launch("tf_w4a16_linear(silu_mul)");
 }
 
 int splitk_reduce(const LinearArgs& a, const float* ws, int split, hipStream_t stream) {
   const bool residual = a.epilogue == TF_EPILOGUE_RESIDUAL;
+  const bool silu = a.epilogue == TF_EPILOGUE_SILU_MUL;
+  const int64_t total = (int64_t)a.m * (silu ? a.n >> 1 : a.n);
   const auto al = [](const void* p, uintptr_t b) { return (reinterpret_cast<uintptr_t>(p) & (b - 1)) == 0; };
-  if (a.epilogue != TF_EPILOGUE_SILU_MUL && split <= kMaxSplitK && (a.n & 3) == 0 && (a.ldo & 3) == 0 &&
-      al(a.out, 8) && al(ws, 16) && (!residual || ((a.ldr & 3) == 0 && al(a.residual, 8)))) {
-    const int64_t runs = (int64_t)a.m * a.n / 4;
-    splitk_reduce4_kernel<<<(unsigned)cdiv(runs, 256), 256, 0, stream>>>(a, ws, split);
+  if (split <= kMaxSplitK && (a.n & (silu ? 7 : 3)) == 0 && (a.ldo & 3) == 0 && al(a.out, 8) && al(ws, 16) &&
+      (!residual || ((a.ldr & 3) == 0 && al(a.residual, 8)))) {
+    const unsigned grid = (unsigned)cdiv(total / 4, 256);
+    if (silu)
+      splitk_reduce4_silu_kernel<<<grid, 256, 0, stream>>>(a, ws, split);
+    else
+      splitk_reduce4_kernel<<<grid, 256, 0, stream>>>(a, ws, split);
     return check_launch("tf_w4a16_linear(splitk_reduce)");
   }
-  const int64_t total = (int64_t)a.m * (a.epilogue == TF_EPILOGUE_SILU_MUL ? a.n >> 1 : a.n);
   splitk_reduce_kernel<<<(unsigned)cdiv(total, 256), 256, 0, stream>>>(a, ws, split);
   return check_launch("tf_w4a16_linear(splitk_reduce)");
 }
 
-// Workspace of an LDS-tile GEMM launch: fp32 partials under split-K, the fp16 y under a
+// Workspace and second kernel of the GEMMs that apply every epilogue themselves: the fp32 partials
+// of a K split and their reduce, else none.
+int64_t split_workspace(const LinearArgs& a, int split) {
+  return split > 1 ? (int64_t)split * a.m * a.n * (int64_t)sizeof(float) : 0;
+}
+
+int finish_split(const LinearArgs& a, const float* ws, int split, hipStream_t stream) {
+  return split > 1 ? splitk_reduce(a, ws, split, stream) : TF_OK;
+}
+
+namespace {
+
+// Workspace of a two-buffer GEMM launch: fp32 partials under split-K, the fp16 y under a
 // SiLU*mul epilogue without split-K, else none.
 int64_t lds_gemm_workspace(const LinearArgs& a, int split) {
   if (split > 1) return (int64_t)split * a.m * a.n * (int64_t)sizeof(float);
@@ -286,14 +356,12 @@ int64_t lds_gemm_workspace(const LinearArgs& a, int split) {
   return 0;
 }
 
-// The kernel after an LDS-tile GEMM launch, if any.
+// The kernel after a two-buffer GEMM launch, if any.
 int lds_gemm_finish(const LinearArgs& a, const float* ws, int split, hipStream_t stream) {
   if (split > 1) return splitk_reduce(a, ws, split, stream);
   if (a.epilogue == TF_EPILOGUE_SILU_MUL) return silu_mul_staged(a, ws, stream);
   return TF_OK;
 }
-
-namespace {
 
 int effective_split(const LinearArgs& a, const tf_gemm_config& cfg) {
   const int nkb = a.k / cfg.block_k;

@@ -48,8 +48,8 @@
 namespace tf {
 
 int splitk_reduce(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
-int64_t lds_gemm_workspace(const LinearArgs& a, int split);
-int lds_gemm_finish(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
+int64_t split_workspace(const LinearArgs& a, int split);
+int finish_split(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
 
 namespace {
 
@@ -116,7 +116,7 @@ __device__ __forceinline__ void block_barrier() {
 // Four-wave 16x16-fragment tiles are compiled for two workgroups per CU (256 registers a
 // wave): their LDS (two x stages, two weight buffers) fits twice, and the two workgroups'
 // barriers then fall at different times.
-template <int BM, int BN, int WM, int WN, int S, int F>
+template <int BM, int BN, int WM, int WN, int S, int F, bool SILU>
 __global__ __launch_bounds__(64 * WM * WN, (WM * WN == 4 && F == 16) ? 2 : 1) void gemm2_kernel(LinearArgs a, float* __restrict__ ws, int split_k,
                                                     int tiles_n, int tiles_m) {
   using C = G2<BM, BN, WM, WN, S, F>;
@@ -191,13 +191,13 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN == 4 && F == 16) ? 2 : 1) vo
     const int id = tid + i * C::kThreads;
     const int col = ((id >> 5) << 4) | (id & 15);
     const int half = (id >> 4) & 1;
-    const int n = n0 + col;
+    const int n = tile_col<SILU>(a, n0, col);
     b_col[i] = col;
     b_half[i] = half;
     const uint32_t tt = (uint32_t)n >> 4, cc = (uint32_t)n & 15u;
     const uint32_t rows = (uint32_t)tile_rows(a.n, tt);
     b_rows[i] = rows;
-    b_off[i] = ((kEvenB || id < C::kBChunks) && n < a.n) ? (tt * q_total * 16u + (uint32_t)half * rows + cc) * 16u
+    b_off[i] = ((kEvenB || id < C::kBChunks) && tile_col_valid<SILU>(a, n0, col)) ? (tt * q_total * 16u + (uint32_t)half * rows + cc) * 16u
                                                           : kOutOfRange;
     b_step[i] = rows * 32u;
     b_sbase[i] = tt * 16u * (uint32_t)groups + cc;
@@ -368,53 +368,11 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN == 4 && F == 16) ? 2 : 1) vo
   }
   if (kb < kb1) iteration(kb, S == 2 ? 0 : st, std::integral_constant<int, 0>{});
 
-  // ---- epilogue. The MFMAs take the weight fragment as their first operand, so each
-  // accumulator tile is y transposed: register q of lane l is row (m) l % F of the tile and
-  // column (n) 4 (l / 16) + q (16x16) or 8 (q / 4) + 4 (l / 32) + q % 4 (32x32). A lane thus
-  // holds runs of four consecutive columns of one row and stores each straight from registers
-  // as one 8-byte piece (fp32 partials: 16 bytes). A SiLU*mul epilogue pairs columns of
-  // different tiles: without split-K the fp16 y goes to the workspace for the SiLU*mul
-  // kernel, with split-K the fp32 partials go to the reduce kernel.
-  const bool partials = split_k > 1;
-  const bool stage_y = !partials && a.epilogue == TF_EPILOGUE_SILU_MUL;
-  uint16_t* const dst = stage_y ? reinterpret_cast<uint16_t*>(ws) : a.out;
-  const int64_t ldd = stage_y ? (int64_t)a.n : a.ldo;
-  const bool residual = !stage_y && a.epilogue == TF_EPILOGUE_RESIDUAL;
-  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
-                           : run_store_ok(a, dst, ldd, residual);
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm) {
-    const int m = m0 + (wm * TM + tm) * F + (lane & (F - 1));
-    if (m >= a.m) continue;
-    const float rs = row_scale(a, m);
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-      for (int g = 0; g < AR / 4; ++g) {
-        const int n = n0 + (wn * TN + tn) * F + (F == 32 ? 8 * g + 4 * (lane >> 5) : 4 * (lane >> 4));
-        if (n >= a.n) continue;
-        float v[4];
-        if (partials) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = acc[tm][tn][4 * g + j];
-          float* const p = ws + ((int64_t)z * a.m + m) * a.n + n;
-          if (vec) {
-            *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (n + j < a.n) p[j] = v[j];
-          }
-          continue;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float b = (a.bias && n + j < a.n) ? half_bits_to_float(a.bias[n + j]) : 0.0f;
-          v[j] = acc[tm][tn][4 * g + j] * rs + b;
-        }
-        store_run4(a, dst, ldd, residual, m, n, v, vec);
-      }
-  }
+  // ---- epilogue (linear.h): runs of four columns straight from the transposed accumulators
+  if constexpr (F == 16)
+    store_tile16<SILU, TM, TN>(a, ws, split_k > 1, z, m0 + wm * TM * F, n0 + wn * TN * F, lane, acc);
+  else
+    store_tile32<SILU, TM, TN>(a, ws, split_k > 1, z, m0 + wm * TM * F, n0 + wn * TN * F, lane, acc);
 }
 
 // ------------------------------------------------------------------ producer / consumer form
@@ -451,7 +409,7 @@ struct G2P {
   static constexpr bool kStreamB = TM * TN > 20;
 };
 
-template <int BM, int BN, int WM, int WN, int S>
+template <int BM, int BN, int WM, int WN, int S, bool SILU>
 __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm2pc_kernel(
     LinearArgs a, float* __restrict__ ws, int split_k, int tiles_n, int tiles_m) {
   using C = G2P<BM, BN, WM, WN, S>;
@@ -515,14 +473,14 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm2pc_kernel(
       const int id = ptid + i * C::kPThreads;
       const int col = ((id >> 5) << 4) | (id & 15);
       const int half = (id >> 4) & 1;
-      const int n = n0 + col;
+      const int n = tile_col<SILU>(a, n0, col);
       b_act[i] = id < C::kBChunks;
       b_col[i] = b_act[i] ? col : 0;
       b_half[i] = half;
       const uint32_t tt = (uint32_t)n >> 4, cc = (uint32_t)n & 15u;
       const uint32_t rows = (uint32_t)tile_rows(a.n, tt);
       b_rows[i] = rows;
-      b_off[i] = (b_act[i] && n < a.n) ? (tt * q_total * 16u + (uint32_t)half * rows + cc) * 16u : kOutOfRange;
+      b_off[i] = (b_act[i] && tile_col_valid<SILU>(a, n0, col)) ? (tt * q_total * 16u + (uint32_t)half * rows + cc) * 16u : kOutOfRange;
       b_step[i] = rows * 32u;
       b_sbase[i] = tt * 16u * (uint32_t)groups + cc;
       b_zbase[i] = tt * 2u * (uint32_t)groups + (cc >> 3);
@@ -651,43 +609,7 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm2pc_kernel(
   }
   if (kb < kb1) iteration(kb, S == 2 ? 0 : st, std::integral_constant<int, 0>{});
 
-  // ---- epilogue (the 16x16 form's, transposed accumulators: see gemm2_kernel)
-  const bool partials = split_k > 1;
-  const bool stage_y = !partials && a.epilogue == TF_EPILOGUE_SILU_MUL;
-  uint16_t* const dst = stage_y ? reinterpret_cast<uint16_t*>(ws) : a.out;
-  const int64_t ldd = stage_y ? (int64_t)a.n : a.ldo;
-  const bool residual = !stage_y && a.epilogue == TF_EPILOGUE_RESIDUAL;
-  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
-                            : run_store_ok(a, dst, ldd, residual);
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm) {
-    const int m = m0 + (wm * TM + tm) * 16 + (lane & 15);
-    if (m >= a.m) continue;
-    const float rs = row_scale(a, m);
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = n0 + (wn * TN + tn) * 16 + 4 * (lane >> 4);
-      if (n >= a.n) continue;
-      float v[4];
-      if (partials) {
-        float* const p = ws + ((int64_t)z * a.m + m) * a.n + n;
-        if (vec) {
-          *reinterpret_cast<f4*>(p) = acc[tm][tn];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (n + j < a.n) p[j] = acc[tm][tn][j];
-        }
-        continue;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float b = (a.bias && n + j < a.n) ? half_bits_to_float(a.bias[n + j]) : 0.0f;
-        v[j] = acc[tm][tn][j] * rs + b;
-      }
-      store_run4(a, dst, ldd, residual, m, n, v, vec);
-    }
-  }
+  store_tile16<SILU, TM, TN>(a, ws, split_k > 1, z, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, acc);
 }
 
 int effective_split2(const LinearArgs& a, const tf_gemm_config& cfg) {
@@ -696,7 +618,7 @@ int effective_split2(const LinearArgs& a, const tf_gemm_config& cfg) {
 }
 
 int64_t gemm2_workspace(const LinearArgs& a, const tf_gemm_config& cfg) {
-  return lds_gemm_workspace(a, effective_split2(a, cfg));
+  return split_workspace(a, effective_split2(a, cfg));
 }
 
 template <int BM, int BN, int WM, int WN, int S, int F>
@@ -709,21 +631,21 @@ int launch_gemm2(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hipS
   if (x_bytes >= (int64_t)kOutOfRange || w_bytes >= (int64_t)kOutOfRange)
     return fail(TF_EINVAL, "tf_w4a16_linear: this gemm_mfma variant needs x and qweight_t below 2 GiB");
   const int split = effective_split2(a, cfg);
-  if (lds_gemm_workspace(a, split) > 0 && ws == nullptr)
+  if (split_workspace(a, split) > 0 && ws == nullptr)
     return fail(TF_EINVAL, "tf_w4a16_linear: this config needs a workspace");
   const int tiles_n = (int)cdiv(a.n, BN);
   const int tiles_m = (int)cdiv(a.m, BM);
   const int64_t grid = (int64_t)tiles_n * tiles_m * split;
   if (grid > 0x7FFFFFFF) return fail(TF_EINVAL, "tf_w4a16_linear: too many tiles");
-  auto kernel = gemm2_kernel<BM, BN, WM, WN, S, F>;
+  const bool silu = split == 1 && a.epilogue == TF_EPILOGUE_SILU_MUL;
+  auto kernel = silu ? gemm2_kernel<BM, BN, WM, WN, S, F, true> : gemm2_kernel<BM, BN, WM, WN, S, F, false>;
   if (C::kLds > 64 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           C::kLds) != hipSuccess)
     return fail(TF_ELAUNCH, "tf_w4a16_linear: cannot reserve LDS for gemm_mfma");
   kernel<<<(unsigned)grid, C::kThreads, C::kLds, stream>>>(a, ws, split, tiles_n, tiles_m);
   if (int rc = check_launch("tf_w4a16_linear(gemm_mfma)")) return rc;
-  return lds_gemm_finish(a, ws, split, stream);
-  return TF_OK;
+  return finish_split(a, ws, split, stream);
 }
 
 template <int BM, int BN, int WM, int WN, int S>
@@ -736,20 +658,21 @@ int launch_gemm2pc(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hi
   if (x_bytes >= (int64_t)kOutOfRange || w_bytes >= (int64_t)kOutOfRange)
     return fail(TF_EINVAL, "tf_w4a16_linear: this gemm_mfma variant needs x and qweight_t below 2 GiB");
   const int split = effective_split2(a, cfg);
-  if (lds_gemm_workspace(a, split) > 0 && ws == nullptr)
+  if (split_workspace(a, split) > 0 && ws == nullptr)
     return fail(TF_EINVAL, "tf_w4a16_linear: this config needs a workspace");
   const int tiles_n = (int)cdiv(a.n, BN);
   const int tiles_m = (int)cdiv(a.m, BM);
   const int64_t grid = (int64_t)tiles_n * tiles_m * split;
   if (grid > 0x7FFFFFFF) return fail(TF_EINVAL, "tf_w4a16_linear: too many tiles");
-  auto kernel = gemm2pc_kernel<BM, BN, WM, WN, S>;
+  const bool silu = split == 1 && a.epilogue == TF_EPILOGUE_SILU_MUL;
+  auto kernel = silu ? gemm2pc_kernel<BM, BN, WM, WN, S, true> : gemm2pc_kernel<BM, BN, WM, WN, S, false>;
   if (C::kLds > 64 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           C::kLds) != hipSuccess)
     return fail(TF_ELAUNCH, "tf_w4a16_linear: cannot reserve LDS for gemm_mfma");
   kernel<<<(unsigned)grid, C::kThreads, C::kLds, stream>>>(a, ws, split, tiles_n, tiles_m);
   if (int rc = check_launch("tf_w4a16_linear(gemm_mfma)")) return rc;
-  return lds_gemm_finish(a, ws, split, stream);
+  return finish_split(a, ws, split, stream);
 }
 
 // num_stages = S + 1 (3: two x stages, 4: three) tells these variants apart from the

@@ -37,8 +37,8 @@
 
 namespace tf {
 
-int64_t lds_gemm_workspace(const LinearArgs& a, int split);
-int lds_gemm_finish(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
+int64_t split_workspace(const LinearArgs& a, int split);
+int finish_split(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
 
 namespace {
 
@@ -104,7 +104,7 @@ __device__ __forceinline__ u2 word_to_e4m3(uint32_t w, const QuantParams& p, con
   return u2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
 }
 
-template <int BM, int BN, int WM, int WN, int S>
+template <int BM, int BN, int WM, int WN, int S, bool SILU>
 __global__ __launch_bounds__(64 * WM * WN) void gemm8_kernel(LinearArgs a, float* __restrict__ ws, int split_k,
                                                     int tiles_n, int tiles_m) {
   using C = G8<BM, BN, WM, WN, S>;
@@ -176,11 +176,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm8_kernel(LinearArgs a, float
     const int id = (tid + i * C::kThreads) % C::kBChunks;
     const int col = ((id >> 6) << 4) | (id & 15);
     const int g = (id >> 4) & 3;
-    const int n = n0 + col;
+    const int n = tile_col<SILU>(a, n0, col);
     b_col[i] = col;
     b_g[i] = g;
     const uint32_t tt = (uint32_t)n >> 4, cc = (uint32_t)n & 15u;
-    const bool ok = n < a.n;
+    const bool ok = tile_col_valid<SILU>(a, n0, col);
     b_off[i] = ok ? (tt * q_total * 16u + (uint32_t)g * 16u + cc) * 16u : kOutOfRange;
     b_sbase[i] = ok ? tt * 16u * (uint32_t)groups + cc : kOutOfRange;
     b_zbase[i] = ok ? tt * 2u * (uint32_t)groups + (cc >> 3) : kOutOfRange;
@@ -300,46 +300,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm8_kernel(LinearArgs a, float
   }
   if (kb < kb1) iteration(kb, S == 2 ? 0 : st, std::integral_constant<int, 0>{});
 
-  // ---- epilogue. The accumulators hold y transposed (weight fragment first): register q of
-  // lane l is row (m) l % 16 and column (n) 4 (l / 16) + q of its tile, so a lane holds a run
-  // of four consecutive columns of one row and stores it as one 8-byte piece (fp32 partials:
-  // 16 bytes) straight from registers.
-  const bool partials = split_k > 1;
-  const bool stage_y = !partials && a.epilogue == TF_EPILOGUE_SILU_MUL;
-  uint16_t* const dst = stage_y ? reinterpret_cast<uint16_t*>(ws) : a.out;
-  const int64_t ldd = stage_y ? (int64_t)a.n : a.ldo;
-  const bool residual = !stage_y && a.epilogue == TF_EPILOGUE_RESIDUAL;
-  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
-                            : run_store_ok(a, dst, ldd, residual);
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm) {
-    const int m = m0 + (wm * TM + tm) * 16 + (lane & 15);
-    if (m >= a.m) continue;
-    const float rs = row_scale(a, m);
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = n0 + (wn * TN + tn) * 16 + 4 * (lane >> 4);
-      if (n >= a.n) continue;
-      float v[4];
-      if (partials) {
-        float* const p = ws + ((int64_t)z * a.m + m) * a.n + n;
-        if (vec) {
-          *reinterpret_cast<f4*>(p) = acc[tm][tn];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (n + j < a.n) p[j] = acc[tm][tn][j];
-        }
-        continue;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float b = (a.bias && n + j < a.n) ? half_bits_to_float(a.bias[n + j]) : 0.0f;
-        v[j] = acc[tm][tn][j] * rs + b;
-      }
-      store_run4(a, dst, ldd, residual, m, n, v, vec);
-    }
-  }
+  store_tile16<SILU, TM, TN>(a, ws, split_k > 1, z, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, acc);
 }
 
 // ------------------------------------------------------------------ producer / consumer form
@@ -370,7 +331,7 @@ struct G8P {
   static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "wave tile");
 };
 
-template <int BM, int BN, int WM, int WN, int S>
+template <int BM, int BN, int WM, int WN, int S, bool SILU>
 __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearArgs a, float* __restrict__ ws,
                                                                          int split_k, int tiles_n, int tiles_m) {
   using C = G8P<BM, BN, WM, WN, S>;
@@ -435,11 +396,11 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearAr
       const int id = (ptid + i * C::kPThreads) % C::kBChunks;
       const int col = ((id >> 6) << 4) | (id & 15);
       const int g = (id >> 4) & 3;
-      const int n = n0 + col;
+      const int n = tile_col<SILU>(a, n0, col);
       b_col[i] = col;
       b_g[i] = g;
       const uint32_t tt = (uint32_t)n >> 4, cc = (uint32_t)n & 15u;
-      const bool ok = n < a.n;
+      const bool ok = tile_col_valid<SILU>(a, n0, col);
       b_off[i] = ok ? (tt * q_total * 16u + (uint32_t)g * 16u + cc) * 16u : kOutOfRange;
       b_sbase[i] = ok ? tt * 16u * (uint32_t)groups + cc : kOutOfRange;
       b_zbase[i] = ok ? tt * 2u * (uint32_t)groups + (cc >> 3) : kOutOfRange;
@@ -547,43 +508,7 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearAr
   }
   if (kb < kb1) iteration(kb, 0, std::integral_constant<int, 0>{});
 
-  // ---- epilogue (gemm8_kernel's)
-  const bool partials = split_k > 1;
-  const bool stage_y = !partials && a.epilogue == TF_EPILOGUE_SILU_MUL;
-  uint16_t* const dst = stage_y ? reinterpret_cast<uint16_t*>(ws) : a.out;
-  const int64_t ldd = stage_y ? (int64_t)a.n : a.ldo;
-  const bool residual = !stage_y && a.epilogue == TF_EPILOGUE_RESIDUAL;
-  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
-                            : run_store_ok(a, dst, ldd, residual);
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm) {
-    const int m = m0 + (wm * TM + tm) * 16 + (lane & 15);
-    if (m >= a.m) continue;
-    const float rs = row_scale(a, m);
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = n0 + (wn * TN + tn) * 16 + 4 * (lane >> 4);
-      if (n >= a.n) continue;
-      float v[4];
-      if (partials) {
-        float* const p = ws + ((int64_t)z * a.m + m) * a.n + n;
-        if (vec) {
-          *reinterpret_cast<f4*>(p) = acc[tm][tn];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (n + j < a.n) p[j] = acc[tm][tn][j];
-        }
-        continue;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float b = (a.bias && n + j < a.n) ? half_bits_to_float(a.bias[n + j]) : 0.0f;
-        v[j] = acc[tm][tn][j] * rs + b;
-      }
-      store_run4(a, dst, ldd, residual, m, n, v, vec);
-    }
-  }
+  store_tile16<SILU, TM, TN>(a, ws, split_k > 1, z, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, acc);
 }
 
 int effective_split8(const LinearArgs& a, const tf_gemm_config& cfg) {
@@ -592,7 +517,7 @@ int effective_split8(const LinearArgs& a, const tf_gemm_config& cfg) {
 }
 
 int64_t gemm8_workspace(const LinearArgs& a, const tf_gemm_config& cfg) {
-  return lds_gemm_workspace(a, effective_split8(a, cfg));
+  return split_workspace(a, effective_split8(a, cfg));
 }
 
 // Everything the launch rejects, before anything is queued.
@@ -617,19 +542,20 @@ int launch_gemm8(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hipS
   using C = G8<BM, BN, WM, WN, S>;
   if (int rc = check_gemm8<BM, BN, WM, WN, S>(a, cfg)) return rc;
   const int split = effective_split8(a, cfg);
-  if (lds_gemm_workspace(a, split) > 0 && ws == nullptr)
+  if (split_workspace(a, split) > 0 && ws == nullptr)
     return fail(TF_EINVAL, "tf_w4a8_linear_ex: this config needs a workspace");
   const int tiles_n = (int)cdiv(a.n, BN);
   const int tiles_m = (int)cdiv(a.m, BM);
   const int64_t grid = (int64_t)tiles_n * tiles_m * split;
-  auto kernel = gemm8_kernel<BM, BN, WM, WN, S>;
+  const bool silu = split == 1 && a.epilogue == TF_EPILOGUE_SILU_MUL;
+  auto kernel = silu ? gemm8_kernel<BM, BN, WM, WN, S, true> : gemm8_kernel<BM, BN, WM, WN, S, false>;
   if (C::kLds > 64 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           C::kLds) != hipSuccess)
     return fail(TF_ELAUNCH, "tf_w4a8_linear_ex: cannot reserve LDS for gemm_fp8");
   kernel<<<(unsigned)grid, C::kThreads, C::kLds, stream>>>(a, ws, split, tiles_n, tiles_m);
   if (int rc = check_launch("tf_w4a8_linear_ex(gemm_fp8)")) return rc;
-  return lds_gemm_finish(a, ws, split, stream);
+  return finish_split(a, ws, split, stream);
 }
 
 template <int BM, int BN, int WM, int WN>
@@ -637,19 +563,20 @@ int launch_gemm8pc(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hi
   using C = G8P<BM, BN, WM, WN, 2>;
   if (int rc = check_gemm8<BM, BN, WM, WN, 2>(a, cfg)) return rc;
   const int split = effective_split8(a, cfg);
-  if (lds_gemm_workspace(a, split) > 0 && ws == nullptr)
+  if (split_workspace(a, split) > 0 && ws == nullptr)
     return fail(TF_EINVAL, "tf_w4a8_linear_ex: this config needs a workspace");
   const int tiles_n = (int)cdiv(a.n, BN);
   const int tiles_m = (int)cdiv(a.m, BM);
   const int64_t grid = (int64_t)tiles_n * tiles_m * split;
-  auto kernel = gemm8pc_kernel<BM, BN, WM, WN, 2>;
+  const bool silu = split == 1 && a.epilogue == TF_EPILOGUE_SILU_MUL;
+  auto kernel = silu ? gemm8pc_kernel<BM, BN, WM, WN, 2, true> : gemm8pc_kernel<BM, BN, WM, WN, 2, false>;
   if (C::kLds > 64 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           C::kLds) != hipSuccess)
     return fail(TF_ELAUNCH, "tf_w4a8_linear_ex: cannot reserve LDS for gemm_fp8");
   kernel<<<(unsigned)grid, C::kThreads, C::kLds, stream>>>(a, ws, split, tiles_n, tiles_m);
   if (int rc = check_launch("tf_w4a8_linear_ex(gemm_fp8)")) return rc;
-  return lds_gemm_finish(a, ws, split, stream);
+  return finish_split(a, ws, split, stream);
 }
 
 // block_k 128 (one group per block); num_stages = S + 1, as the fp16 pipelined GEMM counts them.

@@ -68,6 +68,18 @@ __device__ __forceinline__ bool col_valid(const LinearArgs& a, int n_base, int l
   return silu_out_col(n_base, l) < (a.n >> 1);
 }
 
+// The same mapping for the kernels with an instance for it (SILU: a SiLU*mul call without a K
+// split; with one they write physical columns and the reduce pairs them).
+template <bool SILU>
+__device__ __forceinline__ int tile_col(const LinearArgs& a, int n_base, int l) {
+  if (!SILU) return n_base + l;
+  return ((l & 8) ? a.n >> 1 : 0) + silu_out_col(n_base, l);
+}
+template <bool SILU>
+__device__ __forceinline__ bool tile_col_valid(const LinearArgs& a, int n_base, int l) {
+  return SILU ? silu_out_col(n_base, l) < (a.n >> 1) : n_base + l < a.n;
+}
+
 __device__ __forceinline__ uint16_t f16_bits(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 
 // fp16(residual + fp16(v)): the unfused `residual + linear(x)` of two fp16 tensors.
@@ -127,6 +139,160 @@ __device__ __forceinline__ void store_run4(const LinearArgs& a, uint16_t* dst, i
     uint16_t r = f16_bits(v[j]);
     if (residual) r = finish_residual(v[j], a.residual[(int64_t)m * a.ldr + n + j]);
     dst[(int64_t)m * ldd + n + j] = r;
+  }
+}
+
+// Swaps the upper half wave of a with the lower half wave of b: afterwards lanes 0..31 hold their
+// own a in a and the a of lane + 32 in b, lanes 32..63 the b of lane - 32 in a and their own b in b.
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(as_u32(a), as_u32(b), false, false);
+  a = as_f32(r[0]);
+  b = as_f32(r[1]);
+}
+
+// Columns n .. n + 3 of row m from the sums d of one run: fp32 to slice z of ws [split][M][N]
+// (partials), else y with row scale rs, bias and the NONE / RESIDUAL epilogue to out. vec as in
+// store_run4 (partials: 16-byte pieces of ws).
+__device__ __forceinline__ void store_sums4(const LinearArgs& a, float* ws, bool partials, int z, int m, int n,
+                                            float rs, const f4& d, bool residual, bool vec) {
+  if (partials) {
+    float* const p = ws + ((int64_t)z * a.m + m) * a.n + n;
+    if (vec) {
+      *reinterpret_cast<f4*>(p) = d;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < a.n) p[j] = d[j];
+    }
+    return;
+  }
+  float v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float b = (a.bias && n + j < a.n) ? half_bits_to_float(a.bias[n + j]) : 0.0f;
+    v[j] = d[j] * rs + b;
+  }
+  store_run4(a, a.out, a.ldo, residual, m, n, v, vec);
+}
+
+// Outputs j .. j + 3 of row m under SiLU*mul from the sums of their gate and up columns, one 8-byte
+// piece where vec holds. N % 16 == 0, so a run lies inside N / 2 or past it.
+__device__ __forceinline__ void store_silu4(const LinearArgs& a, int m, int j, float rs, const float (&gate)[4],
+                                            const float (&up)[4], bool vec) {
+  const int half = a.n >> 1;
+  if (j >= half) return;
+  uint16_t h[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float bg = a.bias ? half_bits_to_float(a.bias[j + q]) : 0.0f;
+    const float bu = a.bias ? half_bits_to_float(a.bias[half + j + q]) : 0.0f;
+    // y in fp32 before its fp16 rounding, as the plain epilogue computes it (the empty asm keeps the
+    // compiler from fusing multiply, add and rounding into v_fma_mixlo_f16, which rounds once).
+    float vg = gate[q] * rs + bg, vu = up[q] * rs + bu;
+    __asm__ volatile("" : "+v"(vg), "+v"(vu));
+    h[q] = finish_silu_mul(vg, vu);
+  }
+  uint16_t* const p = a.out + (int64_t)m * a.ldo + j;
+  if (vec) {
+    *reinterpret_cast<u2*>(p) = u2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = h[q];
+  }
+}
+
+// The results of a wave that holds TM x TN transposed 16x16 accumulator tiles (the MFMA with the
+// weight fragment as its first operand): register q of lane l is row (m) l % 16 and column (n)
+// 4 (l / 16) + q of its tile, so a lane holds runs of four consecutive columns of one row. Rows
+// m_base + 16 tm, (virtual) columns n_base + 16 tn.
+// SILU (SiLU*mul without partials): the wave's columns are mapped by phys_col (eight gate columns, then
+// the eight up columns of the same outputs), so lanes l and l + 32 hold the gate and up values of
+// one run. One half-wave swap between the two tiles of a pair gives the lower half wave both
+// values of the first tile and the upper half wave both of the second, and every lane finishes
+// four outputs of each pair. The alternative, fp16 y to a workspace and a second kernel that pairs
+// it, writes and reads [M, N] once more: on MI355X the whole call took 1218 us against 1070 here at
+// gate_up (N 37888, K 3584) M = 4096, 81.3 against 73.9 at M = 256, and 460 against 392 for the fp8
+// GEMM with its norm at M = 2048. An instance of its own (SILU): as a runtime branch it cost the
+// other epilogues 1% (down_proj M = 1000) and spilled the four-wave 32x32 tiles.
+template <bool SILU, int TM, int TN>
+__device__ __forceinline__ void store_tile16(const LinearArgs& a, float* ws, bool partials, int z, int m_base,
+                                             int n_base, int lane, const f4 (&acc)[TM][TN]) {
+  const int g = lane >> 4;
+  if constexpr (SILU) {
+    const int hw = lane >> 5;  // which tile of a pair this lane finishes
+    const bool vec = (a.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      const int m = m_base + tm * 16 + (lane & 15);
+      const float rs = row_scale(a, m);
+#pragma unroll
+      for (int tn = 0; tn < TN; tn += 2) {
+        float gate[4], up[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // every lane takes part, rows past M too
+          gate[q] = acc[tm][tn][q];
+          up[q] = acc[tm][tn + 1 < TN ? tn + 1 : tn][q];
+          swap_halves(gate[q], up[q]);
+        }
+        if (m < a.m && !(tn + 1 >= TN && hw))
+          store_silu4(a, m, (n_base >> 1) + 8 * (tn + hw) + 4 * (g & 1), rs, gate, up, vec);
+      }
+    }
+    return;
+  }
+  const bool residual = a.epilogue == TF_EPILOGUE_RESIDUAL;
+  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
+                            : run_store_ok(a, a.out, a.ldo, residual);
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm) {
+    const int m = m_base + tm * 16 + (lane & 15);
+    if (m >= a.m) continue;
+    const float rs = row_scale(a, m);
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      const int n = n_base + tn * 16 + 4 * g;
+      if (n < a.n) store_sums4(a, ws, partials, z, m, n, rs, acc[tm][tn], residual, vec);
+    }
+  }
+}
+
+// store_tile16 for transposed 32x32 accumulator tiles: register 4 r + q of lane l is row l % 32 and
+// column 8 r + 4 (l / 32) + q, so under the SiLU*mul mapping a lane holds the gate values of a run
+// in registers 8 p .. 8 p + 3 and its up values in 8 p + 4 .. 8 p + 7.
+template <bool SILU, int TM, int TN>
+__device__ __forceinline__ void store_tile32(const LinearArgs& a, float* ws, bool partials, int z, int m_base,
+                                             int n_base, int lane, const f16v (&acc)[TM][TN]) {
+  const int h4 = 4 * (lane >> 5);
+  const bool residual = a.epilogue == TF_EPILOGUE_RESIDUAL;
+  const bool vec = partials ? (a.n & 3) == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0
+                   : SILU   ? (a.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7) == 0
+                            : run_store_ok(a, a.out, a.ldo, residual);
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm) {
+    const int m = m_base + tm * 32 + (lane & 31);
+    if (m >= a.m) continue;
+    const float rs = row_scale(a, m);
+    if constexpr (SILU) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          float gate[4], up[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) gate[q] = acc[tm][tn][8 * p + q], up[q] = acc[tm][tn][8 * p + 4 + q];
+          store_silu4(a, m, (n_base >> 1) + 16 * tn + 8 * p + h4, rs, gate, up, vec);
+        }
+      continue;
+    }
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = n_base + tn * 32 + 8 * r + h4;
+        if (n >= a.n) continue;
+        const f4 d = {acc[tm][tn][4 * r], acc[tm][tn][4 * r + 1], acc[tm][tn][4 * r + 2], acc[tm][tn][4 * r + 3]};
+        store_sums4(a, ws, partials, z, m, n, rs, d, residual, vec);
+      }
   }
 }
 
