@@ -81,6 +81,13 @@ int tf_tile_pack(const int32_t* qweight_t, const uint16_t* scales, const int32_t
                  int32_t* qweight_tile, uint16_t* scales_tile, int32_t* qzeros_tile, int64_t n,
                  int64_t k, int32_t group_size, void* stream);
 
+/* pack.py:171-181 pack_awq in one pass: AWQ qweight [k, n/8], scales and qzeros -> the tile layout
+ * (tf_awq_to_tf, then tf_tile_pack; same bytes). n % 8 == 0, k % group_size == 0; qweight_tile
+ * 16-byte aligned; out-of-place. */
+int tf_awq_to_tile(const int32_t* qweight, const uint16_t* scales, const int32_t* qzeros,
+                   int32_t* qweight_tile, uint16_t* scales_tile, int32_t* qzeros_tile, int64_t n,
+                   int64_t k, int32_t group_size, void* stream);
+
 /* pack.py:184-186 unpack_to_awq (the layout step): exact inverse of tf_tile_pack. */
 int tf_tile_unpack(const int32_t* qweight_tile, const uint16_t* scales_tile,
                    const int32_t* qzeros_tile, int32_t* qweight_t, uint16_t* scales,

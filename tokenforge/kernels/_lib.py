@@ -66,6 +66,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "tf_awq_to_tf": (ctypes.c_int, [_p, _p, _i64, _i64, _p]),
     "tf_tf_to_awq": (ctypes.c_int, [_p, _p, _i64, _i64, _p]),
     "tf_tile_pack": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _p]),
+    "tf_awq_to_tile": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _p]),
     "tf_tile_unpack": (ctypes.c_int, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _p]),
     "tf_awq_quantize": (ctypes.c_int, [_p, _i64, _i64, _i32, _p, _p, _p, _p]),
     "tf_w4a16_dequant": (ctypes.c_int, [_p, _p, _p, _p, _i64, _i64, _i32, _p]),

@@ -136,6 +136,27 @@ def tile_pack(qweight_t: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tenso
     return _tile(qweight_t, scales, qzeros, group_size, to_tile=True)
 
 
+def awq_to_tile(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
+                group_size: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """A validated AWQ layer's ``(qweight, scales, qzeros)`` -> the gfx950 tile layout
+    (``tile_pack(awq_to_tf(qweight), scales, qzeros)``) in one kernel."""
+    if host_route(qweight, scales, qzeros):
+        return host.tile_pack(host.transpose_packed(qweight), scales, qzeros, group_size)
+    run, home = load_time_devices("pack_awq", qweight, scales, qzeros)
+    qw, sc, qz = (t.to(run).contiguous() for t in (qweight, scales, qzeros))
+    dev = require_gpu("pack_awq", qw, sc, qz)
+    k, n8 = qw.shape
+    outs = (torch.empty((n8 * PACK_FACTOR, k // PACK_FACTOR), dtype=torch.int32, device=dev),
+            torch.empty_like(sc), torch.empty_like(qz))
+    if qw.numel():
+        with on_device(dev):
+            rc = _lib.lib().tf_awq_to_tile(qw.data_ptr(), sc.data_ptr(), qz.data_ptr(), outs[0].data_ptr(),
+                                           outs[1].data_ptr(), outs[2].data_ptr(), n8 * PACK_FACTOR, k, group_size,
+                                           stream_of(dev))
+        _lib.check(rc, "pack_awq")
+    return tuple(o.to(home) for o in outs)  # type: ignore[return-value]
+
+
 def tile_unpack(qweight_t: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
                 group_size: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Inverse of :func:`tile_pack`."""

@@ -122,10 +122,10 @@ def validate_awq(
 def pack_awq(
     qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor, group_size: int
 ) -> W4A16Weights:
-    """Load-time conversion of one AWQ layer into the gfx950 tile layout: the GPU repack to the
-    TokenForge layout, then the tile permutation of the weights, scales and zero points."""
+    """Load-time conversion of one AWQ layer into the gfx950 tile layout: the repack to the
+    TokenForge layout and the tile permutation of the weights, scales and zero points, one kernel."""
     validate_awq(qweight, qzeros, scales, group_size)
-    qw, sc, qz = _layout.tile_pack(repack_awq_to_tf(qweight), scales, qzeros, group_size)
+    qw, sc, qz = _layout.awq_to_tile(qweight, scales, qzeros, group_size)
     return W4A16Weights(qweight_t=qw, scales=sc, qzeros=qz, group_size=group_size)
 
 
