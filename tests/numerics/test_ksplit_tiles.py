@@ -1,0 +1,50 @@
+"""The K-split tile GEMM (waves split a tile's K, their sums meet in LDS) against an fp64 product on
+the exact fp16 weights, at the edges of its tiles: M around its rows, N ending inside a tile and
+inside a SiLU*mul column group (N / 16 odd), K shorter than a round of its waves and not a multiple
+of it, every group size, K slices; fused epilogues equal torch's on its own plain output bit for bit,
+and fewer rows per tile change no bit."""
+
+from __future__ import annotations
+
+from dataclasses import replace
+
+import pytest
+import torch
+
+from tests.numerics import cases
+from tokenforge.kernels import pack
+from tokenforge.kernels.config import KSPLIT_TILES, GemmConfig, ksplit_config, ksplit_rows
+from tokenforge.kernels.hip.w4a16 import w4a16_gemm_ex
+
+pytestmark = pytest.mark.gpu
+
+CONFIGS = [ksplit_config(mt, rt, wk) for mt, rt, wk in KSPLIT_TILES]
+
+
+def _id(c: GemmConfig) -> str:
+    return f"{c.block_m}x{c.block_n}-wk{c.waves_k}"
+
+
+@pytest.mark.parametrize("n,k,g,split", [(16, 128, 128, 1), (208, 384, 32, 1), (352, 1152, 64, 1), (336, 2304, 128, 3)])
+@pytest.mark.parametrize("cfg", CONFIGS, ids=_id)
+def test_ksplit_tiles(cfg: GemmConfig, n: int, k: int, g: int, split: int, device: torch.device) -> None:
+    cfg = replace(cfg, split_k=split)
+    w = cases.on_device(cases.layer_weights(n, k, 0, g), device)
+    dense = pack.dequantize_tf(w).double()
+    bias = cases.bias(n, 0).to(device)
+    half = n // 2
+    for m in (1, cfg.block_m - 1, cfg.block_m + 1):
+        x = cases.activations(m, k, 0).to(device)
+        res = cases.activations(m, n, 1).to(device)
+        args = (w.qweight_t, w.scales, w.qzeros, g, cfg, bias)
+        y = w4a16_gemm_ex(x, *args)
+        want = x.double() @ dense.t() + bias.double()
+        # the numerics contract's bound (0.13 sqrt(K) eps max|x| max|w|) above half an fp16 ulp
+        atol = 0.13 * k**0.5 * 2.0**-10 * float(x.abs().max()) * float(dense.abs().max())
+        ulp = torch.ldexp(torch.ones_like(want), torch.frexp(want).exponent.clamp(min=-13) - 12)
+        assert bool(((y.double() - want).abs() <= atol + ulp).all()), f"m={m}"
+        assert torch.equal(w4a16_gemm_ex(x, *args, "residual", res), res + y), f"residual m={m}"
+        silu = torch.nn.functional.silu(y[:, :half]) * y[:, half:]
+        assert torch.equal(w4a16_gemm_ex(x, *args, "silu_mul"), silu), f"silu_mul m={m}"
+        fewer = ksplit_rows(cfg, m)
+        assert torch.equal(w4a16_gemm_ex(x, w.qweight_t, w.scales, w.qzeros, g, fewer, bias), y), f"rows m={m}"

@@ -1,0 +1,50 @@
+"""The launch choice for layers nobody has tuned, on the CPU: every (shape, M, group size) gets a
+config that is compiled and that the library accepts for the shape, the same one whatever the
+epilogue; and a tuned K-split tile keeps its columns and K split when it loses spare rows."""
+
+from __future__ import annotations
+
+import pytest
+
+from tokenforge.kernels.config import KSPLIT_TILES, default_config, ksplit_config, ksplit_rows, m_bucket, untuned_config
+
+SHAPES = [(8, 128), (16, 256), (200, 256), (1000, 1024), (1152, 896), (896, 4864), (2544, 256), (13448, 768), (37888, 3584),
+          (3584, 18944), (4608, 3584), (11040, 5504), (608, 64), (256, 96)]
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize(("n", "k"), SHAPES)
+def test_untuned_configs_run_their_shape(n: int, k: int, group: int) -> None:
+    if k % group:
+        pytest.skip("not a layer")
+    for m in (1, 2, 4, 5, 8, 9, 16, 17, 33, 100, 129, 333, 1000, 4096, 5000):
+        cfg = untuned_config(m, n, k, group)
+        cfg.validate(group)
+        if cfg.ksplit:
+            assert n % 16 == 0 and k % 128 == 0
+            assert cfg.split_k <= k // 128
+        elif cfg.stream:
+            assert m <= cfg.block_m and n % 32 == 0 and k // 128 >= cfg.num_warps
+        elif cfg.kernel == "gemm_mfma" and cfg.block_k == 64:
+            assert group >= 64 or cfg.num_stages == 2
+            assert cfg.split_k <= k // 64
+        else:
+            assert cfg.family == "gemv" or m >= 9
+
+
+def test_rows_of_a_tuned_tile_follow_m() -> None:
+    tuned = ksplit_config(4, 5, 4)
+    assert [ksplit_rows(tuned, m).block_m for m in (1, 16, 33, 48, 49, 64, 65, 90, 100, 128)] == [
+        16, 16, 48, 48, 64, 64, 48, 48, 64, 64]
+    for mt, rt, wk in KSPLIT_TILES:
+        cfg = ksplit_config(mt, rt, wk, 2)
+        for m in (1, 16, 40, 77, 300):
+            got = ksplit_rows(cfg, m)
+            assert (got.block_n, got.waves_k, got.split_k) == (cfg.block_n, cfg.waves_k, cfg.split_k)
+            assert -(-m // got.block_m) == -(-m // cfg.block_m)
+
+
+def test_layers_outside_the_model_keep_the_bucket_default() -> None:
+    for m in (1, 8, 100):
+        assert untuned_config(m, 200, 1024, 128) == default_config(m_bucket(m), 200, 1024, 128)
+    assert untuned_config(64, 1 << 20, 1 << 13, 128) == default_config(64, 1 << 20, 1 << 13, 128)  # 4 GiB of weights

@@ -34,6 +34,9 @@ gemm_mfma  LDS tile M / tile N / tile K K slices across workgroups (fp32 workspa
                                         stages, 6 and 7: the same on 16x16 MFMA fragments
                                         (block_k 64); block_k 128: skinny form, num_stages
                                         = x stages (wave-tile form: 4 + x stages)
+gemm_mfma  tile M (16..128) / tile N /  K slices across workgroups / 8 / 6, 7, 8: 2, 4, 8 of the
+(K split)  128                          waves along K, the rest along N; weights go from memory to the
+                                        MFMA, x through LDS
 gemm_fp8   LDS tile M / tile N / 128    as gemm_mfma (8 waves, num_stages = x stages +
            (one group per block)        1). W4A8 only: e4m3 x on the fp8 MFMA, the group
                                         scale applied in fp32 after each group; chosen by
@@ -46,6 +49,7 @@ Every kernel reads the weights in the gfx950 tile layout that ``pack.pack_awq`` 
 from __future__ import annotations
 
 import functools
+import math
 from dataclasses import asdict, dataclass, replace
 from typing import Any
 
@@ -208,7 +212,24 @@ def _gemm_variants() -> list[tuple[str, int, int, int, int, int]]:
     # wave, WM waves along M), S x stages (x issued S - 1 steps ahead, weights three).
     wave_tiles = [(8, 5, 1, 3), (8, 4, 1, 4), (8, 3, 1, 4), (8, 2, 1, 4)]
     out += [("gemm_mfma", 16 * mt * wm, 16 * rt * (4 // wm), 128, 4, 4 + st) for mt, rt, wm, st in wave_tiles]
+    # block_k 128, eight waves: the K-split tile form, 8 / WK waves along N and WK along K, 16 MT rows
+    # x 16 RT (8 / WK) columns; num_stages 6, 7, 8 for WK = 2, 4, 8.
+    out += [ksplit_config(mt, rt, wk).variant() for mt, rt, wk in KSPLIT_TILES]
     return out
+
+
+KSPLIT_TILES: tuple[tuple[int, int, int], ...] = (
+    (1, 1, 8), (1, 2, 8), (1, 4, 8), (2, 1, 8), (2, 2, 8), (2, 4, 8),
+    (1, 2, 4), (1, 4, 4), (1, 5, 4), (2, 2, 4), (2, 4, 4), (2, 5, 4), (3, 2, 4), (3, 4, 4), (3, 5, 4), (4, 2, 4),
+    (4, 4, 4), (4, 5, 4), (2, 2, 2), (3, 3, 2), (4, 2, 2), (4, 3, 2), (5, 3, 2), (6, 2, 2), (6, 3, 2), (8, 1, 2), (8, 2, 2),
+)
+"""The K-split tile form's (row fragments MT, column tiles per wave RT, waves along K WK), in the
+library's order."""
+
+
+def ksplit_config(mt: int, rt: int, wk: int, split_k: int = 1) -> GemmConfig:
+    """The K-split tile config of 16 ``mt`` rows x 16 ``rt`` (8 / ``wk``) columns."""
+    return GemmConfig("gemm_mfma", 16 * mt, 16 * rt * (8 // wk), 128, split_k, 8, {2: 6, 4: 7, 8: 8}[wk])
 
 
 # W4A8 fp8 GEMM tiles (block_m, block_n, waves along M, waves along N, x stages), in the
@@ -227,13 +248,6 @@ along M, along N), in the library's order after FP8_TILES."""
 def _fp8_variants() -> list[tuple[str, int, int, int, int, int]]:
     return ([("gemm_fp8", bm, bn, 128, wm * wn, s + 1) for bm, bn, wm, wn, s in FP8_TILES]
             + [("gemm_fp8", bm, bn, 128, wm * wn, 8) for bm, bn, wm, wn in FP8_PC_TILES])
-
-
-VARIANTS: tuple[tuple[str, int, int, int, int, int], ...] = tuple(
-    _gemv_variants() + _stream_variants() + _gemm_variants() + _fp8_variants()
-)
-"""(kernel, block_m, block_n, block_k, num_warps, num_stages), in the library's order."""
-_VARIANT_SET = frozenset(VARIANTS)
 
 
 def m_bucket(m: int) -> int:
@@ -268,8 +282,19 @@ class GemmConfig:
 
     @property
     def skinny(self) -> bool:
-        """The skinny gemm_mfma form (block_k 128), which reads each lane's group itself."""
+        """The register-streamed gemm_mfma forms (block_k 128), which read each lane's group
+        themselves."""
         return self.kernel == "gemm_mfma" and self.block_k == 128
+
+    @property
+    def ksplit(self) -> bool:
+        """The K-split tile form of gemm_mfma (block_k 128, eight waves)."""
+        return self.skinny and self.num_warps == 8
+
+    @property
+    def waves_k(self) -> int:
+        """Waves along K of the K-split tile form: num_stages 6, 7, 8 for 2, 4, 8."""
+        return 1 << (self.num_stages - 5)
 
     @property
     def stream(self) -> bool:
@@ -336,6 +361,13 @@ class GemmConfig:
         return cls(**d)
 
 
+VARIANTS: tuple[tuple[str, int, int, int, int, int], ...] = tuple(
+    _gemv_variants() + _stream_variants() + _gemm_variants() + _fp8_variants()
+)
+"""(kernel, block_m, block_n, block_k, num_warps, num_stages), in the library's order."""
+_VARIANT_SET = frozenset(VARIANTS)
+
+
 def _pow2_at_most(v: int, cap: int) -> int:
     p = 1
     while p * 2 <= min(v, cap):
@@ -399,6 +431,165 @@ def default_config(bucket: int, n: int, k: int, group_size: int) -> GemmConfig:
     while tiles * split < NUM_CUS and split * 2 <= min(16, k_blocks):
         split *= 2
     return GemmConfig("gemm_mfma", bm, bn, block_k, split, 4, 2)
+
+
+# ----------------------------------------------------------------------------- untuned launches
+
+def ksplit_applies(n: int, k: int) -> bool:
+    """Whether a layer can run on the K-split tile form: whole 16-column tiles and 128-wide K steps."""
+    return n % 16 == 0 and k % 128 == 0
+
+
+def ksplit_rows(cfg: GemmConfig, m: int) -> GemmConfig:
+    """A K-split tile config with the fewest compiled rows that cover M in as many tiles, its
+    columns and waves along K unchanged (so every sum keeps its order): a bucket's config is tuned
+    at the bucket's M, and rows past M cost LDS reads and MFMAs like any other (gate_up at M = 48 in
+    the bucket of 64: 23.5 us with 48 rows, 25.9 with 64)."""
+    tiles = -(-m // cfg.block_m)
+    rows = [v[1] for v in VARIANTS
+            if v[0] == cfg.kernel and v[2:] == cfg.variant()[2:] and v[1] <= cfg.block_m and -(-m // v[1]) == tiles]
+    return replace(cfg, block_m=min(rows)) if rows else cfg
+
+
+# Time model of the two GEMM forms an untuned layer can run on, fitted (least squares over log
+# time) to 3500 launches on MI355X: ten layer shapes from 1152 x 896 to 37888 x 3584, M = 16 .. 2048,
+# every tile and split of both. Microseconds and bytes:
+#   T = launch + (work^q + hbm^q + l2^q)^(1/q) [+ split], work = rounds over the CUs x time of one
+# workgroup; hbm the layer, x and y once; l2 every workgroup's weights and x. A K-split workgroup runs
+# iterations of MFMAs (MT RT), dequantization (RT) and x (MT WK); a producer/consumer one K blocks of
+# 64 at its tile's rate. The config it picks is 3.4% slower than the best one in the mean over the
+# fitted shapes (at most 29%); the fixed tiles chosen by bucket before were 1.3 to 2.8 times slower.
+_NUM = {
+    "launch": 1.73, "q": 1.66, "hbm": 7.57e6, "split": 2.26, "partials": 8.74e6,
+    "ks_wg": 2.49, "mfma": 0.0836, "dequant": 0.172, "x": 0.0065, "pair": 1.27, "ks_l2": 25.6e6,
+    "pc_wg": 5.53, "pc_block": 0.130, "pc_l2": 17.0e6,
+    # one 64-K block of a tile
+    "pc": {(256, 192): 0.917, (256, 160): 0.803, (256, 128): 0.512, (128, 256): 0.658, (128, 128): 0.192},
+}
+
+
+@functools.lru_cache(maxsize=None)
+def _model_tiles(group_size: int, ksplit: bool) -> tuple[tuple[GemmConfig, float, float, float, bool], ...]:
+    """(config, prologue of a workgroup, time of an iteration or block, rate of its loads, whether two
+    workgroups share a CU) of the model's candidates."""
+    out = []
+    for mt, rt, wk in KSPLIT_TILES if ksplit else ():
+        per_iter = _NUM["mfma"] * mt * rt + _NUM["dequant"] * rt + _NUM["x"] * mt * wk
+        pair = mt * rt <= 4 and rt <= 2 and mt * wk <= 8  # registers and LDS of a second workgroup
+        out.append((ksplit_config(mt, rt, wk), _NUM["ks_wg"], per_iter, _NUM["ks_l2"], pair))
+    if group_size >= 64:
+        for (bm, bn), tile in _NUM["pc"].items():
+            w = 4 if (bm, bn) == (128, 128) else 8
+            out.append((GemmConfig("gemm_mfma", bm, bn, 64, 1, w, 8), _NUM["pc_wg"], _NUM["pc_block"] + tile,
+                        _NUM["pc_l2"], False))
+    return tuple(out)
+
+
+def _model_us(cfg: GemmConfig, costs: tuple[float, float, float, bool], m: int, n: int, k: int) -> float:
+    """Modelled time of ``cfg`` (a row of :func:`_model_tiles` with a split)."""
+    wg_us, iter_us, l2_rate, pair = costs
+    q, split = _NUM["q"], cfg.split_k
+    wgs = -(-m // cfg.block_m) * -(-n // cfg.block_n) * split
+    if pair and wgs > NUM_CUS:
+        rounds = -(-wgs // (2 * NUM_CUS)) * _NUM["pair"]
+    else:
+        rounds = -(-wgs // NUM_CUS)
+    steps = -(-(k // 128) // split)
+    iters = -(-steps // cfg.waves_k) if cfg.ksplit else 2 * steps  # K-split iterations, blocks of 64
+    work = rounds * (wg_us + iters * iter_us)
+    l2 = wgs * (cfg.block_n * 0.53 + cfg.block_m * 2) * (k / split) / l2_rate
+    hbm = (n * k * 0.53 + m * k * 2 + m * n * 2) / _NUM["hbm"]
+    us = (work**q + hbm**q + l2**q) ** (1 / q)
+    return us + (_NUM["split"] + split * m * n * 8 / _NUM["partials"] if split > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _modelled_config(m: int, n: int, k: int, group_size: int) -> tuple[float, GemmConfig] | None:
+    """The modelled time and config of the fastest tile and split (None: no form serves the layer)."""
+    best: tuple[float, GemmConfig] | None = None
+    steps = k // 128
+    for cfg, *costs in _model_tiles(group_size, ksplit_applies(n, k)):
+        if cfg.ksplit and (m <= cfg.block_m - 16 or (-(-m // cfg.block_m) > 4 if m <= 128 else
+                                                     cfg.block_m < 48 or cfg.block_n < 64)):
+            continue  # a smaller tile holds M, or outside the fit: many small tiles refetch the weights
+        tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
+        for split in (1, 2, 3, 4, 6, 8):
+            if split > 1 and (tiles * split > 2 * NUM_CUS or steps < split * (cfg.waves_k if cfg.ksplit else 2)):
+                break
+            split_cfg = replace(cfg, split_k=split)
+            us = _model_us(split_cfg, tuple(costs), m, n, k)
+            if best is None or us < best[0]:
+                best = (us, split_cfg)
+    return best
+
+
+def _model_rows(m: int) -> int:
+    """M rounded up for the model: one evaluation per step of M, not per M."""
+    unit = 16 if m <= 128 else 64 if m <= 1024 else 256
+    return -(-m // unit) * unit
+
+
+RETUNE_MARGIN = 0.93
+"""A tuned K-split tile gives way to the modelled best at this M where the model puts that below
+this share of the tuned tile's time: well inside a bucket the tuned columns can be the wrong ones
+(gate_up in the bucket of 64 is tuned to 64 x 192; at M = 48 48 x 160 takes 23.5 us against 26.6),
+while near the bucket's M the tuner's measurement is the better judge (the model's picks lose 3.4%)."""
+
+
+@functools.lru_cache(maxsize=4096)
+def _retiled(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> GemmConfig:
+    best = _modelled_config(m, n, k, group_size)
+    tiles = {c.variant(): costs for c, *costs in _model_tiles(group_size, True)}
+    if best is None or cfg.variant() not in tiles:
+        return cfg
+    tuned = _model_us(cfg, tuple(tiles[cfg.variant()]), m, n, k)
+    return best[1] if best[0] < RETUNE_MARGIN * tuned else cfg
+
+
+def tuned_at(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> GemmConfig:
+    """The config of a call with M rows whose bucket is tuned to ``cfg``: a K-split tile loses the
+    rows M does not need and, where M is not the bucket's own, may give way to the modelled best."""
+    if not cfg.ksplit:
+        return cfg
+    cfg = ksplit_rows(cfg, m)
+    if m in M_BUCKETS or m > MAX_BUCKET_M or not ksplit_applies(n, k):
+        return cfg
+    return _retiled(cfg, _model_rows(m), n, k, group_size)
+
+
+def untuned_config(m: int, n: int, k: int, group_size: int) -> GemmConfig:
+    """Config of a call with M rows on a layer nobody has tuned (no cache or shipped entry).
+
+    * A layer too large for 32-bit offsets, and up to M = 128 one without whole tiles and K steps:
+      :func:`default_config` of the bucket.
+    * M = 1: the stream form where it is the default (it also runs the norm of
+      ``rmsnorm_fp8_w4a16_linear``), else the K-split GEMV with 16 columns a workgroup and 4 to 16
+      waves by K (896 x 896: 2.9 us against 3.8 with 32 columns).
+    * M <= 8: the stream form where its grid has work for every CU (640 tiles of 16 columns; 16
+      waves from K = 4096 on: 11040 x 5504, M = 3 9.6 us against 10.8 with 8); below that the 16-column
+      GEMV up to M = 4 (3584 x 18944, M = 3: 11.7 us against 17.8) and the tile forms above (M = 8:
+      13.8 us against 22.0).
+    * M > 8: the modelled best of the K-split and the producer/consumer tiles.
+    """
+    bucket = MAX_BUCKET_M if m > MAX_BUCKET_M else m_bucket(m)
+    base = default_config(bucket, n, k, group_size)
+    steps = k // 128
+    ksplit = ksplit_applies(n, k)
+    if n * k // 2 >= 1 << 31 or m * k * 2 >= 1 << 31 or steps < 2 or (not ksplit and m <= 128):
+        return base
+    waves = 4 if steps < 32 else 8 if steps < 56 else 16
+    gemv = GemmConfig("gemv_mfma", 16, 16, 128, 1, min(waves, _pow2_at_most(steps, 16)), 2)
+    if m == 1:
+        return base if base.stream else gemv
+    if m <= STREAM_WIDE_M:
+        form = GemmConfig("gemv_mfma", STREAM_MAX_M if m <= STREAM_MAX_M else STREAM_WIDE_M, 16, STREAM_BLOCK_K, 1,
+                          16 if steps >= 32 else 8, 2)
+        if n >= 640 * 16 and n % 32 == 0 and stream_form_applies(m, n, k, form.num_warps, max_m=form.block_m):
+            return form
+        if m <= STREAM_MAX_M:
+            return gemv
+    best = _modelled_config(_model_rows(m), n, k, group_size)
+    return base if best is None else best[1]
 
 
 def candidate_configs(bucket: int, group_size: int) -> list[GemmConfig]:

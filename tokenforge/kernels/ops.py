@@ -64,12 +64,15 @@ from tokenforge.kernels.config import (
     M_BUCKETS,
     MAX_BUCKET_M,
     NUM_CUS,
+    STREAM_WIDE_M,
     GemmConfig,
     fp8_gemm_applies,
     fp8_gemm_config,
     norm_fused_config,
     split_k_gemv_config,
     stream_form_applies,
+    tuned_at,
+    untuned_config,
 )
 from tokenforge.kernels.device import SUPPORTED_ARCHS, device_arch, gpu_identity
 from tokenforge.kernels.hip import rmsnorm_fp8 as _rms
@@ -123,7 +126,10 @@ def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int) -
     decision = dispatch.select(m, backend="hip", on_gpu=True, triton_ok=runnable,
                                cuda_ext_available=_lib.available())
     dispatch.require_gpu_decision(decision, on_gpu=True)
-    cfg = autotune.lookup(_gpu_id(device), dispatch.lookup_bucket(m), n, k, group_size)
+    key = (_gpu_id(device), dispatch.lookup_bucket(m), n, k, group_size)
+    if autotune.config_source(*key) == "default":
+        return untuned_config(m, n, k, group_size)
+    cfg = tuned_at(autotune.lookup(*key), m, n, k, group_size)
     if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:
         # Above the largest bucket its config is reused; once the M tiles alone fill the CUs a
         # K split only adds the fp32 workspace (split * M * N * 4 bytes) and its reduction.
@@ -151,6 +157,10 @@ def _w4a8_config(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> Ge
     """The W4A8 launch: at prefill M the e4m3 codes go straight into the fp8 MFMA (weights as
     exact e4m3 (q - z), the group scale applied in fp32) instead of being decoded to fp16."""
     bucket = dispatch.lookup_bucket(m)
+    if cfg.ksplit and m <= STREAM_WIDE_M:
+        # The GEMV decodes the codes while it stages x; the tile form would have them converted to
+        # fp16 by a launch of its own.
+        return split_k_gemv_config(n, k)
     if cfg.family == "gemm" and fp8_gemm_applies(bucket, n, k, group_size):
         cfg = fp8_gemm_config(bucket, n, k)
         if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:

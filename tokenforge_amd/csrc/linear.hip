@@ -17,6 +17,8 @@ struct Table {
   int n_gemm3;
   const Variant* gemm4;
   int n_gemm4;
+  const Variant* gemm5;
+  int n_gemm5;
   const Variant* gemm8;
   int n_gemm8;
   Table() {
@@ -26,9 +28,10 @@ struct Table {
     gemm2 = gemm2_variants(&n_gemm2);
     gemm3 = gemm3_variants(&n_gemm3);
     gemm4 = gemm4_variants(&n_gemm4);
+    gemm5 = gemm5_variants(&n_gemm5);
     gemm8 = gemm8_variants(&n_gemm8);
   }
-  int size() const { return n_gemv + n_stream + n_gemm + n_gemm2 + n_gemm3 + n_gemm4 + n_gemm8; }
+  int size() const { return n_gemv + n_stream + n_gemm + n_gemm2 + n_gemm3 + n_gemm4 + n_gemm5 + n_gemm8; }
   const Variant& at(int i) const {
     if (i < n_gemv) return gemv[i];
     i -= n_gemv;
@@ -40,7 +43,9 @@ struct Table {
     i -= n_gemm2;
     if (i < n_gemm3) return gemm3[i];
     i -= n_gemm3;
-    return i < n_gemm4 ? gemm4[i] : gemm8[i - n_gemm4];
+    if (i < n_gemm4) return gemm4[i];
+    i -= n_gemm4;
+    return i < n_gemm5 ? gemm5[i] : gemm8[i - n_gemm5];
   }
 };
 
@@ -71,8 +76,8 @@ int check_config(const tf_gemm_config& cfg, int32_t group_size) {
   const bool stream_form = cfg.kernel == TF_KERNEL_GEMV_MFMA && cfg.block_k == 512;
   if (cfg.kernel != TF_KERNEL_GEMM_MFMA && cfg.kernel != TF_KERNEL_GEMM_FP8 && !stream_form && cfg.split_k != 1)
     return fail(TF_EINVAL, "tf_w4a16_linear: gemv kernels split K across waves (num_warps); split_k must be 1");
-  // block_k 128 marks the skinny kernel (gemm3.hip), which reads each lane's group itself;
-  // the LDS-tile kernels need one scale per column and block.
+  // block_k 128 marks the register-streamed kernels (gemm3.hip, gemm4.hip, gemm5.hip), which read each
+  // lane's group themselves; the LDS-tile kernels need one scale per column and block.
   if (cfg.kernel == TF_KERNEL_GEMM_MFMA && cfg.block_k != 128 &&
       (cfg.block_k > group_size || group_size % cfg.block_k))
     return fail(TF_EINVAL, "tf_w4a16_linear: block_k must divide group_size");
