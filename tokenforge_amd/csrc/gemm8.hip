@@ -362,10 +362,13 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearAr
 
   if (producer) {
     const int groups = a.k >> a.log2g;  // == nkb (group_size 128)
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x8, (uint32_t)((int64_t)(a.m - 1) * a.ldx8 + a.k));
-    const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.qw, (uint32_t)((int64_t)a.n * (a.k >> 1)));
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)(groups * a.n * 2));
-    const __amdgpu_buffer_rsrc_t rz = make_rsrc(a.qz, (uint32_t)(groups * (a.n >> 3) * 4));
+    // Buffer sizes: a block past the K range is loaded through an empty resource (wave-uniform, zeros);
+    // inside it the block's offset is scalar, so a producer spends no VALU on addresses (gate_up M =
+    // 2048 on MI355X with its norm: 386 us against 391 with per-lane offsets and range selects).
+    const uint32_t x_bytes = (uint32_t)((int64_t)(a.m - 1) * a.ldx8 + a.k);
+    const uint32_t q_bytes = (uint32_t)((int64_t)a.n * (a.k >> 1));
+    const uint32_t s_bytes = (uint32_t)(groups * a.n * 2);
+    const uint32_t z_bytes = (uint32_t)(groups * (a.n >> 3) * 4);
     const UnpackConsts uc = unpack_consts();
     uint32_t a_off[C::kAPerWave];
 #pragma unroll
@@ -376,21 +379,24 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearAr
       const int m = m0 + row;
       a_off[i] = m < a.m ? (uint32_t)((int64_t)m * a.ldx8 + c * 16) : kOutOfRange;
     }
-    auto issue_a = [&](int kb, int st) {
+    auto issue_a = [&](int kb, int st) __attribute__((always_inline)) {
       const bool ok = kb < kb1;
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x8, ok ? x_bytes : 0u);
+      const int32_t soff = ok ? kb * kBK : 0;
 #pragma unroll
       for (int i = 0; i < C::kAPerWave; ++i) {
-        const uint32_t off = ok ? a_off[i] + (uint32_t)kb * kBK : kOutOfRange;
+        const uint32_t off = a_off[i];
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rx, (__attribute__((address_space(3))) void*)(a_lds + st * C::kAStage + (pwave + C::kProd * i) * 1024), 16,
-            off, 0, 0, 0);
+            off, soff, 0, 0);
       }
     };
     // chunk (ptid + i * producers) % chunks, as gemm8_kernel assigns them (a few producer
     // threads redo a chunk another one converts: same data to the same place)
     const uint32_t q_total = (uint32_t)(a.k >> 5);
     uint32_t b_off[BP], b_sbase[BP], b_zbase[BP];
-    int b_col[BP], b_g[BP];
+    uint32_t b_zsh[BP];
+    int b_col[BP], b_lds_off[BP];
 #pragma unroll
     for (int i = 0; i < BP; ++i) {
       const int id = (ptid + i * C::kPThreads) % C::kBChunks;
@@ -398,34 +404,38 @@ __global__ __launch_bounds__(64 * (WM * WN + 4), 1) void gemm8pc_kernel(LinearAr
       const int g = (id >> 4) & 3;
       const int n = tile_col<SILU>(a, n0, col);
       b_col[i] = col;
-      b_g[i] = g;
+      b_lds_off[i] = (int)swz8(col, 2 * g);  // the odd chunk: ^ 16
+      b_zsh[i] = 4u * awq_nibble_of((uint32_t)n & 7u);
       const uint32_t tt = (uint32_t)n >> 4, cc = (uint32_t)n & 15u;
       const bool ok = tile_col_valid<SILU>(a, n0, col);
       b_off[i] = ok ? (tt * q_total * 16u + (uint32_t)g * 16u + cc) * 16u : kOutOfRange;
-      b_sbase[i] = ok ? tt * 16u * (uint32_t)groups + cc : kOutOfRange;
-      b_zbase[i] = ok ? tt * 2u * (uint32_t)groups + (cc >> 3) : kOutOfRange;
+      b_sbase[i] = ok ? (tt * 16u * (uint32_t)groups + cc) * 2u : kOutOfRange;
+      b_zbase[i] = ok ? (tt * 2u * (uint32_t)groups + (cc >> 3)) * 4u : kOutOfRange;
     }
     u4 braw[2][BP];
     uint32_t bsc[2][BP], bzw[2][BP];
-    auto issue_b = [&](int kb, int slot) {
+    auto issue_b = [&](int kb, int slot) __attribute__((always_inline)) {
       const bool ok = kb < kb1;
+      const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.qw, ok ? q_bytes : 0u);
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, ok ? s_bytes : 0u);
+      const __amdgpu_buffer_rsrc_t rz = make_rsrc(a.qz, ok ? z_bytes : 0u);
+      const int sb = ok ? kb : 0;
 #pragma unroll
       for (int i = 0; i < BP; ++i) {
-        const bool v = ok && b_off[i] != kOutOfRange;
-        braw[slot][i] = load_b128(rq, v ? b_off[i] + (uint32_t)kb * 1024u : kOutOfRange);
-        bsc[slot][i] = load_b16(rs, v ? (b_sbase[i] + (uint32_t)kb * 16u) * 2u : kOutOfRange);
-        bzw[slot][i] = load_b32(rz, v ? (b_zbase[i] + (uint32_t)kb * 2u) * 4u : kOutOfRange);
+        braw[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rq, (int)b_off[i], sb * 1024, 0);
+        bsc[slot][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs, (int)b_sbase[i], sb * 32, 0);
+        bzw[slot][i] = __builtin_amdgcn_raw_buffer_load_b32(rz, (int)b_zbase[i], sb * 8, 0);
       }
     };
     auto store_b = [&](int slot, int buf) {
 #pragma unroll
       for (int i = 0; i < BP; ++i) {
-        const QuantParams qp = make_params(zero_of(bzw[slot][i], (uint32_t)(n0 + b_col[i])), bsc[slot][i]);
+        const QuantParams qp = make_params((bzw[slot][i] >> b_zsh[i]) & 0xFu, bsc[slot][i]);
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
           const u2 lo = word_to_e4m3(braw[slot][i][2 * part], qp, uc);
           const u2 hi = word_to_e4m3(braw[slot][i][2 * part + 1], qp, uc);
-          *reinterpret_cast<u4*>(b_lds + buf * C::kBStage + swz8(b_col[i], 2 * b_g[i] + part)) =
+          *reinterpret_cast<u4*>(b_lds + buf * C::kBStage + (b_lds_off[i] ^ (16 * part))) =
               u4{lo[0], lo[1], hi[0], hi[1]};
         }
         s_lds[buf * BN + b_col[i]] = half_bits_to_float((uint16_t)bsc[slot][i]);
