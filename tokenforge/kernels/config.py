@@ -435,6 +435,11 @@ def default_config(bucket: int, n: int, k: int, group_size: int) -> GemmConfig:
 
 # ----------------------------------------------------------------------------- untuned launches
 
+SPAN_32BIT = 1 << 31
+"""Bytes of x and of the packed weights from which on only the two-buffer GEMM (num_stages 2) runs: the
+other kernels address both through 32-bit buffer offsets."""
+
+
 def ksplit_applies(n: int, k: int) -> bool:
     """Whether a layer can run on the K-split tile form: whole 16-column tiles and 128-wide K steps."""
     return n % 16 == 0 and k % 128 == 0
@@ -557,11 +562,13 @@ def tuned_at(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> GemmCo
     return _retiled(cfg, _model_rows(m), n, k, group_size)
 
 
-def untuned_config(m: int, n: int, k: int, group_size: int) -> GemmConfig:
+def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) -> GemmConfig:
     """Config of a call with M rows on a layer nobody has tuned (no cache or shipped entry).
+    ``x_bytes``: the bytes from x's first element to its last, for rows with a stride of their own.
 
-    * A layer too large for 32-bit offsets, and up to M = 128 one without whole tiles and K steps:
-      :func:`default_config` of the bucket.
+    * A layer or an x too large for 32-bit offsets, and up to M = 128 a layer without whole tiles and
+      K steps: :func:`default_config` of the bucket (for groups of 32 the two-buffer GEMM, which
+      addresses both in 64 bits).
     * M = 1: the stream form where it is the default (it also runs the norm of
       ``rmsnorm_fp8_w4a16_linear``), else the K-split GEMV with 16 columns a workgroup and 4 to 16
       waves by K (896 x 896: 2.9 us against 3.8 with 32 columns).
@@ -575,7 +582,7 @@ def untuned_config(m: int, n: int, k: int, group_size: int) -> GemmConfig:
     base = default_config(bucket, n, k, group_size)
     steps = k // 128
     ksplit = ksplit_applies(n, k)
-    if n * k // 2 >= 1 << 31 or m * k * 2 >= 1 << 31 or steps < 2 or (not ksplit and m <= 128):
+    if n * k // 2 >= SPAN_32BIT or max(m * k * 2, x_bytes) >= SPAN_32BIT or steps < 2 or (not ksplit and m <= 128):
         return base
     waves = 4 if steps < 32 else 8 if steps < 56 else 16
     gemv = GemmConfig("gemv_mfma", 16, 16, 128, 1, min(waves, _pow2_at_most(steps, 16)), 2)

@@ -116,8 +116,9 @@ def _record_host(m: int, backend: str) -> None:
     dispatch.record(dispatch.select(m, backend=backend, on_gpu=False))  # type: ignore[arg-type]
 
 
-def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int) -> GemmConfig:
-    """The launch config of a call with M rows on ``device`` (after the device check).
+def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int, x_bytes: int = 0) -> GemmConfig:
+    """The launch config of a call with M rows on ``device`` (after the device check); ``x_bytes`` as
+    in :func:`config.untuned_config`.
 
     A ``torch_reference`` decision here (library missing, other GPU) raises: GPU tensors never
     fall back. The tuned config may pick the other kernel family in the buckets both serve.
@@ -128,7 +129,7 @@ def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int) -
     dispatch.require_gpu_decision(decision, on_gpu=True)
     key = (_gpu_id(device), dispatch.lookup_bucket(m), n, k, group_size)
     if autotune.config_source(*key) == "default":
-        return untuned_config(m, n, k, group_size)
+        return untuned_config(m, n, k, group_size, x_bytes)
     cfg = tuned_at(autotune.lookup(*key), m, n, k, group_size)
     if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:
         # Above the largest bucket its config is reused; once the M tiles alone fill the CUs a
@@ -145,10 +146,10 @@ def _family(cfg: GemmConfig) -> dispatch.Kernel:
     return "hip_gemm" if cfg.family == "gemm" else "hip_gemv"
 
 
-def _decide(x2: torch.Tensor, m: int, n: int, k: int, group_size: int, backend: str) -> GemmConfig:
+def _decide(x2: torch.Tensor, m: int, n: int, k: int, group_size: int, backend: str, x_bytes: int = 0) -> GemmConfig:
     """Dispatch decision and launch config of a call on GPU tensors (the Python body's path);
     the counter records the family that runs."""
-    cfg = _gpu_config(x2.device, m, n, k, group_size)
+    cfg = _gpu_config(x2.device, m, n, k, group_size, x_bytes)
     dispatch.record(dispatch.Decision(_family(cfg), dispatch.bucket_label(m)))
     return cfg
 
@@ -264,7 +265,7 @@ def _linear(
         _, _, _, bias, r2 = _w4a16.check_linear_args(x2, qweight_t, scales, qzeros, group_size, bias, epilogue, r2)
         _record_host(m, backend)
         return host.linear(x2, qweight_t, scales, qzeros, bias, group_size, epilogue, r2).reshape(out_shape)
-    cfg = _decide(x2, m, n, k, group_size, backend)
+    cfg = _decide(x2, m, n, k, group_size, backend, ((m - 1) * x2.stride(0) + k) * 2)
     y = _w4a16.w4a16_gemm_ex(x2, qweight_t, scales, qzeros, group_size, cfg, bias, epilogue, r2)
     return y.reshape(out_shape)
 

@@ -262,6 +262,9 @@ at::Tensor linear_fast(int64_t epi, const at::Tensor& x, const at::Tensor& qw, c
   if (m == 0 || n == 0 || x.scalar_type() != at::kHalf || !weights_ok(qw, sc, qz, k, g, dev) || !bias_ok(bias, n, dev))
     return {};
   if (epi == TF_EPILOGUE_SILU_MUL && n % 16 != 0) return {};
+  // Rows so far apart that x spans more than the cached config's 32-bit offsets: the Python body
+  // chooses with the stride in hand.
+  if (m > 1 && ((m - 1) * x2.stride(0) + k) * 2 > 0x7FFFFFFF && m * k * 2 <= 0x7FFFFFFF) return {};
   at::Tensor r2;
   if (epi == TF_EPILOGUE_RESIDUAL) {
     const at::Tensor& r = *residual;
