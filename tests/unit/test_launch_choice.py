@@ -1,0 +1,35 @@
+"""The operators' launch choice (resolver and Python body) on the CPU, for an MI355X that is not there:
+what each call would launch and what its dispatch counter says."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tokenforge.kernels import _lib, ops
+from tokenforge.kernels.metrics import KERNEL_CALLS
+
+FAMILY_OF = {_lib.KERNEL_IDS[k]: ("hip_gemm" if k in ("gemm_mfma", "gemm_fp8") else "hip_gemv") for k in _lib.KERNEL_IDS}
+DEV = torch.device("cuda", 0)
+
+
+@pytest.fixture(autouse=True)
+def _mi355x(monkeypatch: pytest.MonkeyPatch) -> None:
+    monkeypatch.setattr(ops, "device_arch", lambda device: "gfx950")
+    monkeypatch.setattr(ops, "_gpu_id", lambda device: "amd-gfx950-256cu")
+    KERNEL_CALLS.reset()
+
+
+@pytest.mark.parametrize("kind", [ops.KIND_LINEAR, ops.KIND_W4A8, ops.KIND_NORM_LINEAR])
+@pytest.mark.parametrize(("n", "k", "g"), [(896, 896, 64), (3584, 3584, 128), (37888, 3584, 128), (1152, 4096, 32)])
+def test_the_counter_names_the_family_that_runs(kind: int, n: int, k: int, g: int) -> None:
+    for m in (1, 3, 5, 8, 9, 16, 17, 100, 300):
+        fields = ops._resolve_launch(kind, _lib.EPILOGUE_NONE, m, n, k, g, 0)
+        assert ops._FAMILIES[fields[7]] == FAMILY_OF[fields[0]], f"m={m}"
+        if kind == ops.KIND_NORM_LINEAR:
+            continue
+        before = {lab: KERNEL_CALLS.value(kernel=lab, bucket=ops._BUCKET_LABELS[fields[8]]) for lab in ops._FAMILIES}
+        cfg = ops._decide(DEV, m, n, k, g, w4a8=kind == ops.KIND_W4A8)
+        after = {lab: KERNEL_CALLS.value(kernel=lab, bucket=ops._BUCKET_LABELS[fields[8]]) for lab in ops._FAMILIES}
+        assert {lab: after[lab] - before[lab] for lab in after} == {
+            lab: int(lab == ops._family(cfg)) for lab in after}, f"m={m}"

@@ -146,10 +146,13 @@ def _family(cfg: GemmConfig) -> dispatch.Kernel:
     return "hip_gemm" if cfg.family == "gemm" else "hip_gemv"
 
 
-def _decide(x2: torch.Tensor, m: int, n: int, k: int, group_size: int, backend: str, x_bytes: int = 0) -> GemmConfig:
+def _decide(device: torch.device, m: int, n: int, k: int, group_size: int, x_bytes: int = 0,
+            w4a8: bool = False) -> GemmConfig:
     """Dispatch decision and launch config of a call on GPU tensors (the Python body's path);
     the counter records the family that runs."""
-    cfg = _gpu_config(x2.device, m, n, k, group_size, x_bytes)
+    cfg = _gpu_config(device, m, n, k, group_size, x_bytes)
+    if w4a8:
+        cfg = _w4a8_config(cfg, m, n, k, group_size)
     dispatch.record(dispatch.Decision(_family(cfg), dispatch.bucket_label(m)))
     return cfg
 
@@ -186,7 +189,6 @@ def _resolve_launch(kind: int, epilogue: int, m: int, n: int, k: int, group_size
     the norm + linear, whether the GEMV's prologue runs the norm."""
     dev = torch.device("cuda", device)
     cfg = _gpu_config(dev, m, n, k, group_size)
-    family = _FAMILIES.index(_family(cfg))
     fused = 0
     h = _lib.lib()
     if kind == KIND_W4A8:
@@ -200,6 +202,7 @@ def _resolve_launch(kind: int, epilogue: int, m: int, n: int, k: int, group_size
                 cfg, fused = fcfg, 1
         c = _w4a16.to_c_config(cfg)
         need = 0 if fused else int(h.tf_w4a16_workspace_bytes_ex(m, n, k, group_size, ctypes.byref(c), epilogue))
+    family = _FAMILIES.index(_family(cfg))
     bucket = _BUCKET_LABELS.index(dispatch.bucket_label(m))
     return [c.kernel, c.block_m, c.block_n, c.block_k, c.split_k, c.num_warps, c.num_stages, family, bucket, need,
             fused]
@@ -265,7 +268,7 @@ def _linear(
         _, _, _, bias, r2 = _w4a16.check_linear_args(x2, qweight_t, scales, qzeros, group_size, bias, epilogue, r2)
         _record_host(m, backend)
         return host.linear(x2, qweight_t, scales, qzeros, bias, group_size, epilogue, r2).reshape(out_shape)
-    cfg = _decide(x2, m, n, k, group_size, backend, ((m - 1) * x2.stride(0) + k) * 2)
+    cfg = _decide(x2.device, m, n, k, group_size, ((m - 1) * x2.stride(0) + k) * 2)
     y = _w4a16.w4a16_gemm_ex(x2, qweight_t, scales, qzeros, group_size, cfg, bias, epilogue, r2)
     return y.reshape(out_shape)
 
@@ -321,7 +324,7 @@ def _w4a8_linear(x8, x_scale, qweight_t, scales, qzeros, bias, group_size, backe
         _record_host(m, backend)
         y = host.w4a8_linear(x2, x_scale.reshape(-1), qweight_t, scales, qzeros, bias, group_size, epilogue, r2)
         return y.reshape(out_shape)
-    cfg = _w4a8_config(_decide(x2, m, n, k, group_size, backend), m, n, k, group_size)
+    cfg = _decide(x2.device, m, n, k, group_size, w4a8=True)
     # One contiguous scale vector: the kernel reads its data pointer with the stride of this view.
     s2 = (x_scale.reshape(-1) if x_scale.numel() > 1 else x_scale.reshape(1)).contiguous()
     r2 = residual.reshape(-1, n) if residual is not None else None
@@ -427,7 +430,7 @@ def _rmsnorm_fp8_w4a16_linear(x, norm_weight, eps, qweight_t, scales, qzeros, bi
         _, _, _, bias, _ = _w4a16.check_linear_args(a, qweight_t, scales, qzeros, group_size, bias, epilogue, None)
         _record_host(m, backend)
         return host.linear(a, qweight_t, scales, qzeros, bias, group_size, epilogue).reshape(out_shape)
-    cfg = _decide(x2, m, n, k, group_size, backend)
+    cfg = _decide(x2.device, m, n, k, group_size)
     fcfg = norm_fused_config(cfg, m, n, k)
     if fcfg is not None:
         y = _w4a16.rmsnorm_fp8_w4a16_gemm_ex(
