@@ -33,3 +33,15 @@ def test_the_counter_names_the_family_that_runs(kind: int, n: int, k: int, g: in
         after = {lab: KERNEL_CALLS.value(kernel=lab, bucket=ops._BUCKET_LABELS[fields[8]]) for lab in ops._FAMILIES}
         assert {lab: after[lab] - before[lab] for lab in after} == {
             lab: int(lab == ops._family(cfg)) for lab in after}, f"m={m}"
+
+
+@pytest.mark.parametrize(("n", "k", "one_launch"), [
+    (3584, 3584, True), (896, 896, True), (9728, 896, True), (4096, 4096, True), (4112, 3584, False),
+    (9728, 1536, False), (3584, 4224, False), (37888, 3584, False)])
+def test_w4a8_up_to_16_rows_decodes_while_staging_where_that_is_faster(n: int, k: int, one_launch: bool) -> None:
+    for m in (9, 12, 16):
+        cfg = ops._decide(DEV, m, n, k, 128, w4a8=True)
+        assert (cfg.family == "gemv") == one_launch, f"m={m}: {cfg}"
+        if one_launch:
+            assert ops._resolve_launch(ops.KIND_W4A8, _lib.EPILOGUE_NONE, m, n, k, 128, 0)[9] == 0  # no workspace
+    assert ops._decide(DEV, 17, n, k, 128, w4a8=True).ksplit

@@ -669,6 +669,28 @@ def fp8_gemm_applies(bucket: int, n: int, k: int, group_size: int) -> bool:
     return bucket >= FP8_MIN_BUCKET and group_size == 128 and k % 128 == 0 and n % 16 == 0
 
 
+W4A8_GEMV_MAX_M = 16
+"""Rows of one tile of the 16-column GEMV, up to which it may replace a K-split tile in a W4A8 call."""
+
+
+def w4a8_gemv_config(m: int, n: int, k: int) -> GemmConfig | None:
+    """The GEMV that a W4A8 call of M rows runs where its W4A16 config is a K-split tile, or None where
+    the tile is the faster one. The GEMV decodes the codes while it stages x; the tile form has them
+    converted to fp16 by a launch of its own (about 2 us).
+
+    Up to M = 8: the form that runs every shape. Up to M = 16: 16 columns and 4 to 16 waves a workgroup
+    where that is one round over the CUs (16 waves with their rows of x take a CU's LDS) and K is at most
+    4096. Measured on MI355X at M = 12, conversion included, GEMV / tile: 3584 x 3584 7.5 / 8.3 us, 896 x
+    896 5.0 / 6.1, 9728 x 896 6.1 / 8.3; two rounds 4608 x 3584 13.1 / 10.3, 9728 x 1536 10.8 / 9.5; long
+    K 3584 x 5632 10.2 / 10.1, 3584 x 11008 15.3 / 13.7."""
+    if m <= STREAM_WIDE_M:
+        return split_k_gemv_config(n, k)
+    waves = _pow2_at_most(k // 128, 16)
+    if m <= W4A8_GEMV_MAX_M and k <= 4096 and -(-n // 16) * waves <= 16 * NUM_CUS:
+        return GemmConfig("gemv_mfma", 16, 16, 128, 1, waves, 2)
+    return None
+
+
 # Makespan model of the fp8 GEMM on MI355X (fit to its measured times on the Qwen2.5-7B shapes):
 # a workgroup runs one 128-K block of a BM x BN tile at about 4.2 TFLOP/s, the 256 x 160 tile 5%
 # slower per FLOP; a K split adds about 3 us plus its fp32 partials (split * M * N * 4 bytes

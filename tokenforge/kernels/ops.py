@@ -64,7 +64,6 @@ from tokenforge.kernels.config import (
     M_BUCKETS,
     MAX_BUCKET_M,
     NUM_CUS,
-    STREAM_WIDE_M,
     GemmConfig,
     fp8_gemm_applies,
     fp8_gemm_config,
@@ -73,6 +72,7 @@ from tokenforge.kernels.config import (
     stream_form_applies,
     tuned_at,
     untuned_config,
+    w4a8_gemv_config,
 )
 from tokenforge.kernels.device import SUPPORTED_ARCHS, device_arch, gpu_identity
 from tokenforge.kernels.hip import rmsnorm_fp8 as _rms
@@ -161,10 +161,8 @@ def _w4a8_config(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> Ge
     """The W4A8 launch: at prefill M the e4m3 codes go straight into the fp8 MFMA (weights as
     exact e4m3 (q - z), the group scale applied in fp32) instead of being decoded to fp16."""
     bucket = dispatch.lookup_bucket(m)
-    if cfg.ksplit and m <= STREAM_WIDE_M:
-        # The GEMV decodes the codes while it stages x; the tile form would have them converted to
-        # fp16 by a launch of its own.
-        return split_k_gemv_config(n, k)
+    if cfg.ksplit and (gemv := w4a8_gemv_config(m, n, k)) is not None:
+        return gemv
     if cfg.family == "gemm" and fp8_gemm_applies(bucket, n, k, group_size):
         cfg = fp8_gemm_config(bucket, n, k)
         if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:
