@@ -45,3 +45,13 @@ def test_w4a8_up_to_16_rows_decodes_while_staging_where_that_is_faster(n: int, k
         if one_launch:
             assert ops._resolve_launch(ops.KIND_W4A8, _lib.EPILOGUE_NONE, m, n, k, 128, 0)[9] == 0  # no workspace
     assert ops._decide(DEV, 17, n, k, 128, w4a8=True).ksplit
+
+
+@pytest.mark.parametrize(("n", "k", "g"), [(1000, 1024, 32), (4096, 4096, 128), (5760, 2944, 32), (3584, 18944, 128)])
+def test_no_k_split_once_the_row_tiles_fill_the_cus(n: int, k: int, g: int) -> None:
+    for m in (4097, 9000, 20000, 70000):
+        cfg = ops._gpu_config(DEV, m, n, k, g)
+        tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
+        assert cfg.split_k == 1 or tiles < 256, f"m={m}: {cfg}"
+        need = ops._resolve_launch(ops.KIND_LINEAR, _lib.EPILOGUE_NONE, m, n, k, g, 0)[9]
+        assert (need == 0) == (cfg.split_k == 1), f"m={m}"

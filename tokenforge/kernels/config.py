@@ -567,8 +567,8 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     ``x_bytes``: the bytes from x's first element to its last, for rows with a stride of their own.
 
     * A layer or an x too large for 32-bit offsets, and up to M = 128 a layer without whole tiles and
-      K steps: :func:`default_config` of the bucket (for groups of 32 the two-buffer GEMM, which
-      addresses both in 64 bits).
+      K steps: :func:`default_config` of the bucket. Past 2 GiB the library runs only the two-buffer
+      GEMM among these (M > 128 in groups of 32) and refuses the others, whose offsets are 32-bit.
     * M = 1: the stream form where it is the default (it also runs the norm of
       ``rmsnorm_fp8_w4a16_linear``), else the K-split GEMV with 16 columns a workgroup and 4 to 16
       waves by K (896 x 896: 2.9 us against 3.8 with 32 columns).
