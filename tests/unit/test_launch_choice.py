@@ -6,7 +6,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from tokenforge.kernels import _lib, ops
+from tokenforge.kernels import _lib, autotune, ops
+from tokenforge.kernels.config import ksplit_config, ksplit_rows
 from tokenforge.kernels.metrics import KERNEL_CALLS
 
 FAMILY_OF = {_lib.KERNEL_IDS[k]: ("hip_gemm" if k in ("gemm_mfma", "gemm_fp8") else "hip_gemv") for k in _lib.KERNEL_IDS}
@@ -55,3 +56,11 @@ def test_no_k_split_once_the_row_tiles_fill_the_cus(n: int, k: int, g: int) -> N
         assert cfg.split_k == 1 or tiles < 256, f"m={m}: {cfg}"
         need = ops._resolve_launch(ops.KIND_LINEAR, _lib.EPILOGUE_NONE, m, n, k, g, 0)[9]
         assert (need == 0) == (cfg.split_k == 1), f"m={m}"
+
+
+def test_an_entry_of_the_callers_own_cache_keeps_its_tile() -> None:
+    n, k, g = 37888, 3584, 128
+    shipped = ops._gpu_config(DEV, 80, n, k, g)
+    own = ksplit_config(4, 5, 4)
+    autotune.get_cache("amd-gfx950-256cu").put(128, n, k, g, own)
+    assert ops._gpu_config(DEV, 80, n, k, g) == ksplit_rows(own, 80) != shipped

@@ -6,7 +6,15 @@ from __future__ import annotations
 
 import pytest
 
-from tokenforge.kernels.config import KSPLIT_TILES, default_config, ksplit_config, ksplit_rows, m_bucket, untuned_config
+from tokenforge.kernels.config import (
+    KSPLIT_TILES,
+    default_config,
+    ksplit_config,
+    ksplit_rows,
+    m_bucket,
+    tuned_at,
+    untuned_config,
+)
 
 SHAPES = [(8, 128), (16, 256), (200, 256), (1000, 1024), (1152, 896), (896, 4864), (2544, 256), (13448, 768), (37888, 3584),
           (3584, 18944), (4608, 3584), (11040, 5504), (608, 64), (256, 96)]
@@ -48,3 +56,25 @@ def test_layers_outside_the_model_keep_the_bucket_default() -> None:
     for m in (1, 8, 100):
         assert untuned_config(m, 200, 1024, 128) == default_config(m_bucket(m), 200, 1024, 128)
     assert untuned_config(64, 1 << 20, 1 << 13, 128) == default_config(64, 1 << 20, 1 << 13, 128)  # 4 GiB of weights
+
+
+def test_a_tuned_tile_gives_way_inside_its_bucket_only() -> None:
+    gate_up = (37888, 3584, 128)
+    tuned64, tuned128 = ksplit_config(4, 3, 2), ksplit_config(4, 5, 4)
+    for m in range(49, 65):  # the model's rows are the bucket's: the tuner measured these tiles
+        assert tuned_at(tuned64, m, *gate_up) == tuned64
+    assert tuned_at(tuned128, 80, *gate_up) == ksplit_config(5, 3, 2)  # one tile of 80 rows against two of 48
+    for m in (9, 33, 65, 80, 100, 127):  # a choice of the caller's own tuner only loses spare rows
+        for cfg in (tuned64, tuned128):
+            assert tuned_at(cfg, m, *gate_up, own=True) == ksplit_rows(cfg, m)
+
+
+def test_tuned_choices_fit_their_layer() -> None:
+    for n, k in ((37888, 3584), (4608, 3584), (3584, 3584), (3584, 18944), (256, 1024)):
+        for mt, rt, wk in KSPLIT_TILES:
+            for m in (9, 20, 40, 70, 100, 129, 200, 300, 500):
+                for split in (1, 4):
+                    cfg = tuned_at(ksplit_config(mt, rt, wk, split), m, n, k, 128)
+                    cfg.validate(128)
+                    assert not cfg.ksplit or (n % 16 == 0 and k % 128 == 0)
+                    assert cfg.split_k <= k // 64

@@ -128,10 +128,11 @@ def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int, x
                                cuda_ext_available=_lib.available())
     dispatch.require_gpu_decision(decision, on_gpu=True)
     key = (_gpu_id(device), dispatch.lookup_bucket(m), n, k, group_size)
-    if autotune.config_source(*key) == "default":
+    source = autotune.config_source(*key)
+    if source == "default":
         cfg = untuned_config(m, n, k, group_size, x_bytes)
     else:
-        cfg = tuned_at(autotune.lookup(*key), m, n, k, group_size)
+        cfg = tuned_at(autotune.lookup(*key), m, n, k, group_size, own=source == "cache")
     if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:
         # Above the largest bucket its config is reused; once the M tiles alone fill the CUs a
         # K split only adds the fp32 workspace (split * M * N * 4 bytes) and its reduction.
