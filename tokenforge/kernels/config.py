@@ -566,6 +566,28 @@ def tuned_at(cfg: GemmConfig, m: int, n: int, k: int, group_size: int, own: bool
     return _retiled(cfg, _model_rows(m), n, k, group_size)
 
 
+def _narrow_decode_config(m: int, n: int, k: int, base: GemmConfig) -> GemmConfig:
+    """The M <= 4 choice between ``base``, the bucket's default (the stream form, or the 32-column GEMV
+    where that does not run), and the GEMV with 16 columns a workgroup.
+
+    Against the stream form at M = 1 base; at M = 2 .. 4 the GEMV up to K = 2048, with 4 waves up to K =
+    1024 and 8 above (M = 3, GEMV / stream: 2048 x 1024 4.0 / 4.3 us, 4608 x 2048 5.3 / 6.1; longer K
+    4096 x 2944 6.1 / 5.4, 5120 x 11008 15.2 / 13.7, 4608 x 4096 8.1 / 7.4). Against the 32-column GEMV:
+    while its workgroups are one round over the CUs (N <= 4096) always, with 4, 8 or 16 waves by K (528
+    x 4096, M = 3 5.3 / 7.0; 3584 x 18944 11.7 / 17.8); past that 4 waves below K = 4096 and 64M
+    weights and 8 up to K = 8192 (6160 x 8192 11.6 / 12.3; 4608 x 18944 24.5 / 20.9, 16400 x 4096 14.8 /
+    14.4, 20432 x 3840 at M = 4 18.8 / 16.5). Over 800 calls of 1 to 8 rows on 140 random layers the choice
+    took 0.78 of the default's time in the mean, at most 1.04."""
+    steps = k // 128
+    if base.stream:
+        waves = 0 if m == 1 or steps > 16 else 4 if steps <= 8 else 8
+    elif n <= 16 * NUM_CUS:
+        waves = 4 if steps < 32 else 8 if steps < 56 else 16
+    else:
+        waves = (4 if n * k <= 64 << 20 else 0) if steps < 32 else 8 if steps <= 64 and n < 640 * 16 else 0
+    return GemmConfig("gemv_mfma", 16, 16, 128, 1, min(waves, _pow2_at_most(steps, 16)), 2) if waves else base
+
+
 def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) -> GemmConfig:
     """Config of a call with M rows on a layer nobody has tuned (no cache or shipped entry).
     ``x_bytes``: the bytes from x's first element to its last, for rows with a stride of their own.
@@ -573,13 +595,11 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     * A layer or an x too large for 32-bit offsets, and up to M = 128 a layer without whole tiles and
       K steps: :func:`default_config` of the bucket. Past 2 GiB the library runs only the two-buffer
       GEMM among these (M > 128 in groups of 32) and refuses the others, whose offsets are 32-bit.
-    * M = 1: the stream form where it is the default (it also runs the norm of
-      ``rmsnorm_fp8_w4a16_linear``), else the K-split GEMV with 16 columns a workgroup and 4 to 16
-      waves by K (896 x 896: 2.9 us against 3.8 with 32 columns).
-    * M <= 8: the stream form where its grid has work for every CU (640 tiles of 16 columns; 16
-      waves from K = 4096 on: 11040 x 5504, M = 3 9.6 us against 10.8 with 8); below that the 16-column
-      GEMV up to M = 4 (3584 x 18944, M = 3: 11.7 us against 17.8) and the tile forms above (M = 8:
-      13.8 us against 22.0).
+    * M <= 8, at least 640 tiles of 16 columns (work for every CU): the stream form where it runs, with 16
+      waves from K = 4096 on (11040 x 5504, M = 3 9.6 us against 10.8 with 8).
+    * M <= 4 below that: :func:`_narrow_decode_config`.
+    * M = 5 .. 8: a wide layer of few weights as at M <= 4 (K too short for the stream form: 17712 x 256
+      4.4 us against 5.7 for the tile), the others the modelled tile (512 x 4096 5.6 us against 8.2).
     * M > 8: the modelled best of the K-split and the producer/consumer tiles.
     """
     bucket = MAX_BUCKET_M if m > MAX_BUCKET_M else m_bucket(m)
@@ -588,17 +608,13 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     ksplit = ksplit_applies(n, k)
     if n * k // 2 >= SPAN_32BIT or max(m * k * 2, x_bytes) >= SPAN_32BIT or steps < 2 or (not ksplit and m <= 128):
         return base
-    waves = 4 if steps < 32 else 8 if steps < 56 else 16
-    gemv = GemmConfig("gemv_mfma", 16, 16, 128, 1, min(waves, _pow2_at_most(steps, 16)), 2)
-    if m == 1:
-        return base if base.stream else gemv
-    if m <= STREAM_WIDE_M:
+    if 1 < m <= STREAM_WIDE_M and n >= 640 * 16 and n % 32 == 0:
         form = GemmConfig("gemv_mfma", STREAM_MAX_M if m <= STREAM_MAX_M else STREAM_WIDE_M, 16, STREAM_BLOCK_K, 1,
                           16 if steps >= 32 else 8, 2)
-        if n >= 640 * 16 and n % 32 == 0 and stream_form_applies(m, n, k, form.num_warps, max_m=form.block_m):
+        if stream_form_applies(m, n, k, form.num_warps, max_m=form.block_m):
             return form
-        if m <= STREAM_MAX_M:
-            return gemv
+    if m <= STREAM_MAX_M or (m <= STREAM_WIDE_M and n >= 640 * 16 and n * k <= 12 << 20):
+        return _narrow_decode_config(m, n, k, base)
     best = _modelled_config(_model_rows(m), n, k, group_size)
     return base if best is None else best[1]
 
