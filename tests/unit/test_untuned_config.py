@@ -91,3 +91,13 @@ def test_decode_rows_keep_the_default_where_it_is_faster(n: int, k: int, m: int,
         assert cfg == default_config(m_bucket(m), n, k, 128)
     else:
         assert (cfg.kernel, cfg.block_k, (cfg.block_n, cfg.num_warps)) == ("gemv_mfma", 128, kernel)
+
+
+@pytest.mark.parametrize(("n", "k", "m", "tile"), [
+    (4096, 4096, 3584, (256, 256)), (11008, 4096, 1025, (256, 256)), (2048, 8192, 8000, (256, 256)),
+    (5760, 2944, 2560, (256, 256)), (5760, 2944, 1300, (256, 160)), (11008, 4096, 2048, (256, 192)),
+])
+def test_prefill_takes_the_tile_with_the_fewest_rounds(n: int, k: int, m: int, tile: tuple[int, int]) -> None:
+    cfg = untuned_config(m, n, k, 128)
+    assert (cfg.block_m, cfg.block_n, cfg.split_k) == (*tile, 1)
+    assert cfg.num_stages == (3 if tile == (256, 256) else 8)

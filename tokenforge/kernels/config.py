@@ -470,6 +470,8 @@ _NUM = {
     "pc_wg": 5.53, "pc_block": 0.130, "pc_l2": 17.0e6,
     # one 64-K block of a tile
     "pc": {(256, 192): 0.917, (256, 160): 0.803, (256, 128): 0.512, (128, 256): 0.658, (128, 128): 0.192},
+    # the shared-role 256 x 256 tile, fitted to 880 launches above M = 256 beside the others' model
+    "wide_wg": 7.0, "wide_block": 1.52,
 }
 
 
@@ -487,6 +489,10 @@ def _model_tiles(group_size: int, ksplit: bool) -> tuple[tuple[GemmConfig, float
             w = 4 if (bm, bn) == (128, 128) else 8
             out.append((GemmConfig("gemm_mfma", bm, bn, 64, 1, w, 8), _NUM["pc_wg"], _NUM["pc_block"] + tile,
                         _NUM["pc_l2"], False))
+        # Slower per column than the producer/consumer tiles but wider than any of them: the fewest
+        # rounds where its tiles fill one or two (4096 x 4096 M = 3584 124 us, 256 x 128 133).
+        out.append((GemmConfig("gemm_mfma", 256, 256, 64, 1, 8, 3), _NUM["wide_wg"], _NUM["wide_block"], _NUM["pc_l2"],
+                    False))
     return tuple(out)
 
 
@@ -600,7 +606,7 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     * M <= 4 below that: :func:`_narrow_decode_config`.
     * M = 5 .. 8: a wide layer of few weights as at M <= 4 (K too short for the stream form: 17712 x 256
       4.4 us against 5.7 for the tile), the others the modelled tile (512 x 4096 5.6 us against 8.2).
-    * M > 8: the modelled best of the K-split and the producer/consumer tiles.
+    * M > 8: the modelled best of the K-split, the producer/consumer and the 256 x 256 tiles.
     """
     bucket = MAX_BUCKET_M if m > MAX_BUCKET_M else m_bucket(m)
     base = default_config(bucket, n, k, group_size)
