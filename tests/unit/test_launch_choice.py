@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from tokenforge.kernels import _lib, autotune, ops
-from tokenforge.kernels.config import ksplit_config, ksplit_rows
+from tokenforge.kernels.config import fill_split, ksplit_config, ksplit_rows
 from tokenforge.kernels.metrics import KERNEL_CALLS
 
 FAMILY_OF = {_lib.KERNEL_IDS[k]: ("hip_gemm" if k in ("gemm_mfma", "gemm_fp8") else "hip_gemv") for k in _lib.KERNEL_IDS}
@@ -64,3 +64,9 @@ def test_an_entry_of_the_callers_own_cache_keeps_its_tile() -> None:
     own = ksplit_config(4, 5, 4)
     autotune.get_cache("amd-gfx950-256cu").put(128, n, k, g, own)
     assert ops._gpu_config(DEV, 80, n, k, g) == ksplit_rows(own, 80) != shipped
+
+
+def test_down_proj_at_256_rows_fills_the_cus_once() -> None:
+    cfg = ops._gpu_config(DEV, 256, 3584, 18944, 128)
+    assert (cfg.block_m, cfg.block_n, cfg.num_stages) == (256, 128, 8)
+    assert cfg.split_k == fill_split(cfg, 256, 3584, 18944) == 9
