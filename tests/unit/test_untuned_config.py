@@ -1,11 +1,15 @@
 """The launch choice for layers nobody has tuned, on the CPU: every (shape, M, group size) gets a
-config that is compiled and that the library accepts for the shape, the same one whatever the
-epilogue; and a tuned K-split tile keeps its columns and K split when it loses spare rows."""
+config that the library has compiled, allows for the group size and whose kernel serves the shape
+(its N, K and M conditions, restated here), the same one whatever the epilogue; and a tuned K-split
+tile keeps its columns and K split when it loses spare rows."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 
+from tokenforge.kernels import _lib
 from tokenforge.kernels.config import (
     KSPLIT_TILES,
     default_config,
@@ -15,6 +19,7 @@ from tokenforge.kernels.config import (
     tuned_at,
     untuned_config,
 )
+from tokenforge.kernels.hip.w4a16 import to_c_config
 
 SHAPES = [(8, 128), (16, 256), (200, 256), (1000, 1024), (1152, 896), (896, 4864), (2544, 256), (13448, 768), (37888, 3584),
           (3584, 18944), (4608, 3584), (11040, 5504), (608, 64), (256, 96)]
@@ -28,6 +33,11 @@ def test_untuned_configs_run_their_shape(n: int, k: int, group: int) -> None:
     for m in (1, 2, 4, 5, 8, 9, 16, 17, 33, 100, 129, 333, 1000, 4096, 5000):
         cfg = untuned_config(m, n, k, group)
         cfg.validate(group)
+        # without rows the library checks the sizes and the config and returns
+        c = to_c_config(cfg)
+        rc = _lib.lib().tf_w4a16_linear_ex(None, k, None, None, None, None, None, n, 0, n, k, group, ctypes.byref(c), 0,
+                                           None, 0, None, 0, None)
+        assert rc == 0, f"m={m}: {cfg}"
         if cfg.ksplit:
             assert n % 16 == 0 and k % 128 == 0
             assert cfg.split_k <= k // 128
@@ -55,7 +65,8 @@ def test_rows_of_a_tuned_tile_follow_m() -> None:
 def test_layers_outside_the_model_keep_the_bucket_default() -> None:
     for m in (1, 8, 100):
         assert untuned_config(m, 200, 1024, 128) == default_config(m_bucket(m), 200, 1024, 128)
-    assert untuned_config(64, 1 << 20, 1 << 13, 128) == default_config(64, 1 << 20, 1 << 13, 128)  # 4 GiB of weights
+    assert untuned_config(64, 1 << 20, 1 << 13, 128) == default_config(64, 1 << 20, 1 << 13, 128)
+    # ... 4 GiB of weights, which the library refuses at this M: the form's offsets are 32-bit
 
 
 def test_a_tuned_tile_gives_way_inside_its_bucket_only() -> None:
