@@ -13,6 +13,7 @@ import pytest
 from tests.unit.test_isa_order import CSRC, _instructions, _order_after_barriers, _wait_checks
 from tokenforge_amd import build
 
+X_STAGES = 2
 _KERNEL = re.compile(r"^(_Z\w*gemm5_kernelI(\w*?)EEv\w*):")
 
 
@@ -35,8 +36,7 @@ def test_ksplit_stage_waits(tmp_path: Path) -> None:
         if not m:
             continue
         end = next(j for j in range(i + 1, len(lines)) if lines[j].startswith(".Lfunc_end"))
-        stages = [int(v) for v in re.findall(r"Li(\d+)E", m.group(2) + "E")][4]
-        rows = _wait_checks(_instructions(lines[i + 1:end]), stages)
+        rows = _wait_checks(_instructions(lines[i + 1:end]), X_STAGES)
         assert len(rows) >= 2, m.group(1)
         for b, n, after in rows:
             assert after >= 0 and after != float("inf"), f"{m.group(1)}: barrier at {b}"

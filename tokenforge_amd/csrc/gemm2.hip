@@ -47,7 +47,6 @@
 
 namespace tf {
 
-int splitk_reduce(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
 int64_t split_workspace(const LinearArgs& a, int split);
 int finish_split(const LinearArgs& a, const float* ws, int split, hipStream_t stream);
 

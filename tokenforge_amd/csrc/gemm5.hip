@@ -23,9 +23,10 @@
 //
 // LDS rows hold 16 chunks of 16 bytes (one 256-byte bank line); chunk c of row r sits in slot
 // c ^ (r & 11), free of bank conflicts for the fragment reads (lane 16 g + c at row c, chunk
-// 4 g + j), as in gemm4.hip. Loads of steps past the workgroup's K range go through an empty buffer
-// resource (zeros), so every wave issues the same loads in every iteration and the barrier's
-// vmcnt wait stays exact. Shapes: N % 16 == 0, K % 128 == 0.
+// 4 g + j), as in gemm4.hip. Steps past the workgroup's K range are loaded all the same, as zeros
+// (weights through an empty buffer resource, x at an offset out of range), so every wave issues the
+// same loads in every iteration and the barrier's vmcnt wait stays exact. Shapes: N % 16 == 0, K %
+// 128 == 0.
 //
 // Split-K over workgroups (split_k > 1): K slices write fp32 partials [split][M][N] to the caller's
 // workspace and splitk_reduce (gemm.hip) sums them in split order.
@@ -42,7 +43,7 @@ namespace {
 
 constexpr int kStepK = 128;
 
-template <int MT, int RT, int WN, int WK, int S, int P>
+template <int MT, int RT, int WN, int WK, int P>
 struct G5 {
   static constexpr int kWaves = WN * WK;
   static constexpr int kThreads = 64 * kWaves;
@@ -51,17 +52,15 @@ struct G5 {
   static constexpr int kSub = BM * kStepK * 2;                     // bytes of one step of x
   static constexpr int kStage = WK * kSub;                         // bytes of one x stage
   static constexpr int kDma = kStage / 1024;                       // 1 KB LDS-load instructions per stage
-  static constexpr int kDmaPerWave = (kDma + kWaves - 1) / kWaves;  // (spare ones fill the dummy KB)
-  static constexpr bool kEven = kDma % kWaves == 0;
+  static constexpr int kDmaPerWave = kDma / kWaves;
   static constexpr int kSums = kWaves * MT * RT * 1024;  // the partial sums that meet in LDS
-  static constexpr int kX = S * kStage + (kEven ? 0 : 1024);
-  static constexpr int kLds = WK > 1 && kSums > kX ? kSums : kX;
-  // VMEM issued after x stage t (S - 1 iterations back) when iteration t waits for it: the weights
-  // issued at that iteration's end, then S - 2 whole iterations. (The first iterations may have more
-  // in flight; their wait is then longer, never too short.)
-  static constexpr int kAfterX = 3 * RT + (S - 2) * (kDmaPerWave + 3 * RT);
-  static_assert(kWaves == 8, "eight waves");
-  static_assert(S >= 2 && S <= 3, "x stages");
+  static constexpr int kLds = kSums > 2 * kStage ? kSums : 2 * kStage;
+  // VMEM issued after x stage t (an iteration back) when iteration t waits for it: the weights issued
+  // at that iteration's end. (The first iterations may have more in flight; their wait is then longer,
+  // never too short.)
+  static constexpr int kAfterX = 3 * RT;
+  static_assert(kWaves == 8 && WK >= 2, "eight waves, at least two of them along K");
+  static_assert(kDma % kWaves == 0, "every wave loads the same share of a stage");
   static_assert(P >= 2 && P <= 4, "register ring of two to four steps");
   static_assert(kLds <= 160 * 1024, "x stages or sums exceed the LDS");
   static_assert(kAfterX < 64, "vmcnt range");
@@ -76,10 +75,10 @@ __device__ __forceinline__ void step_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int MT, int RT, int WN, int WK, int S, int P, bool SILU>
+template <int MT, int RT, int WN, int WK, int P, bool SILU>
 __global__ __launch_bounds__(64 * WN * WK, 2) void gemm5_kernel(LinearArgs a, float* __restrict__ ws, int split_k,
                                                                 int tiles_n, int tiles_m) {
-  using C = G5<MT, RT, WN, WK, S, P>;
+  using C = G5<MT, RT, WN, WK, P>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
   const int tid = threadIdx.x;
@@ -118,7 +117,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm5_kernel(LinearArgs a, fl
     const int i = wave + C::kWaves * ii;
     const int sub = i / (4 * MT);
     const int row = 4 * (i - sub * 4 * MT) + g;
-    x_sub[ii] = C::kEven || i < C::kDma ? sub : 0x10000;  // a spare instruction is never inside K
+    x_sub[ii] = sub;
     x_off[ii] = m0 + row < a.m
                     ? (uint32_t)(((int64_t)(m0 + row) * a.ldx + (int64_t)sub * kStepK + (c ^ (row & 11)) * 8) * 2)
                     : kOutOfRange;
@@ -129,7 +128,7 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm5_kernel(LinearArgs a, fl
       const int i = wave + C::kWaves * ii;
       const bool ok = s + x_sub[ii] < s1;  // wave-uniform
       const uint32_t off = ok ? x_off[ii] + (uint32_t)s * (kStepK * 2) : kOutOfRange;
-      const uint32_t dst = C::kEven || i < C::kDma ? (uint32_t)(st * C::kStage + i * 1024) : (uint32_t)(S * C::kStage);
+      const uint32_t dst = (uint32_t)(st * C::kStage + i * 1024);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(smem + dst), 16, off, 0, 0,
                                                0);
     }
@@ -217,9 +216,8 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm5_kernel(LinearArgs a, fl
     }
   };
 
-  // ---- prologue: x stages 0 .. S - 2 in flight, weights of this wave's first P steps in the ring
-#pragma unroll
-  for (int i = 0; i < S - 1; ++i) issue_x(s0 + i * WK, i);
+  // ---- prologue: the first x stage in flight, weights of this wave's first P steps in the ring
+  issue_x(s0, 0);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < P; ++i) {
@@ -227,58 +225,52 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm5_kernel(LinearArgs a, fl
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // Iteration at stage start s (ring slot a compile-time value): wait for its x stage, issue the
-  // stage S - 1 ahead into the one read in the previous iteration, multiply this wave's step, refill
-  // its ring slot. In the tail (fewer than P stages left) the weights an iteration issues are never
+  // Iteration at stage start s (ring slot a compile-time value): wait for its x stage, issue the next
+  // one into the stage read in the previous iteration, multiply this wave's step, refill its ring slot. In the tail (fewer than P stages left) the weights an iteration issues are never
   // read, so the compiler drops those loads and the count after the stage is smaller than kAfterX:
   // the tail's barriers wait for every load instead.
   auto iteration = [&](int s, int st, auto slot_tag, auto tail_tag) __attribute__((always_inline)) {
     constexpr int slot = decltype(slot_tag)::value;
     step_barrier<decltype(tail_tag)::value ? 0 : C::kAfterX>();
-    issue_x(s + (S - 1) * WK, st + S - 1 < S ? st + S - 1 : st - 1);
+    issue_x(s + WK, 1 - st);
     // The waits count the loads issued after each x stage: no later load may move above it.
     __builtin_amdgcn_sched_barrier(0);
     if (s + kz < s1) compute(st, slot);  // wave-uniform: no step left for this wave past the end
     issue_w(s + kz + P * WK, slot);
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto next = [](int st) { return st + 1 == S ? 0 : st + 1; };
   using Loop = std::false_type;
   using Tail = std::true_type;
   int s = s0, st = 0;
   for (; s + (P - 1) * WK < s1; s += P * WK) {
     iteration(s, st, std::integral_constant<int, 0>{}, Loop{});
-    st = next(st);
+    st = 1 - st;
     iteration(s + WK, st, std::integral_constant<int, 1>{}, Loop{});
-    st = next(st);
+    st = 1 - st;
     if constexpr (P > 2) {
       iteration(s + 2 * WK, st, std::integral_constant<int, 2>{}, Loop{});
-      st = next(st);
+      st = 1 - st;
     }
     if constexpr (P > 3) {
       iteration(s + 3 * WK, st, std::integral_constant<int, 3>{}, Loop{});
-      st = next(st);
+      st = 1 - st;
     }
   }
   // Fewer than P stages remain.
   if (s < s1) {
     iteration(s, st, std::integral_constant<int, 0>{}, Tail{});
-    st = next(st);
+    st = 1 - st;
   }
   if constexpr (P > 2) {
     if (s + WK < s1) {
       iteration(s + WK, st, std::integral_constant<int, 1>{}, Tail{});
-      st = next(st);
+      st = 1 - st;
     }
   }
   if constexpr (P > 3) {
     if (s + 2 * WK < s1) iteration(s + 2 * WK, st, std::integral_constant<int, 2>{}, Tail{});
   }
 
-  if constexpr (WK == 1) {
-    store_tile16<SILU, MT, RT>(a, ws, split_k > 1, z, m0, 16 * v0, lane, acc);
-    return;
-  }
   // ---- the WK partial sums of each tile, through LDS (every x stage has been read; the loads
   // still in flight are of stages past the end: the barrier waits until they have landed, before
   // their LDS is reused): wave (wn, kz) takes row tiles kz, kz + WK, ... and adds them in kz order.
@@ -331,16 +323,16 @@ int check_gemm5(const LinearArgs& a, const tf_gemm_config& cfg) {
   return TF_OK;
 }
 
-template <int MT, int RT, int WN, int WK, int S, int P>
+template <int MT, int RT, int WN, int WK, int P>
 int launch_gemm5(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hipStream_t stream) {
-  using C = G5<MT, RT, WN, WK, S, P>;
+  using C = G5<MT, RT, WN, WK, P>;
   if (int rc = check_gemm5<C::BM, C::BN>(a, cfg)) return rc;
   const int split = effective_split5(a, cfg);
   if (split > 1 && ws == nullptr) return fail(TF_EINVAL, "tf_w4a16_linear: split-K needs a workspace");
   const int tiles_n = (int)cdiv(a.n, C::BN);
   const int tiles_m = (int)cdiv(a.m, C::BM);
   const bool silu = split == 1 && a.epilogue == TF_EPILOGUE_SILU_MUL;
-  auto kernel = silu ? gemm5_kernel<MT, RT, WN, WK, S, P, true> : gemm5_kernel<MT, RT, WN, WK, S, P, false>;
+  auto kernel = silu ? gemm5_kernel<MT, RT, WN, WK, P, true> : gemm5_kernel<MT, RT, WN, WK, P, false>;
   if (int rc = reserve_lds(kernel, C::kLds, "gemm_mfma")) return rc;
   kernel<<<(unsigned)(tiles_n * tiles_m * split), C::kThreads, C::kLds, stream>>>(a, ws, split, tiles_n, tiles_m);
   if (int rc = check_launch("tf_w4a16_linear(gemm_mfma)")) return rc;
@@ -351,7 +343,7 @@ int launch_gemm5(const LinearArgs& a, const tf_gemm_config& cfg, float* ws, hipS
 // or 8 for WK = 2, 4 or 8 waves along K.
 #define TF_GEMM5(MT, RT, WN, WK, P)                                                        \
   {{TF_KERNEL_GEMM_MFMA, 16 * MT, 16 * RT * WN, 128, 1, WN * WK, WK == 2 ? 6 : WK == 4 ? 7 : 8}, \
-   (launch_gemm5<MT, RT, WN, WK, 2, P>), gemm5_workspace, (check_gemm5<16 * MT, 16 * RT * WN>)}
+   (launch_gemm5<MT, RT, WN, WK, P>), gemm5_workspace, (check_gemm5<16 * MT, 16 * RT * WN>)}
 
 const Variant kGemm5Variants[] = {
     // WK 8: narrow tiles, K split over all eight waves
