@@ -70,3 +70,10 @@ def test_down_proj_at_256_rows_fills_the_cus_once() -> None:
     cfg = ops._gpu_config(DEV, 256, 3584, 18944, 128)
     assert (cfg.block_m, cfg.block_n, cfg.num_stages) == (256, 128, 8)
     assert cfg.split_k == fill_split(cfg, 256, 3584, 18944) == 9
+
+
+def test_gate_up_keeps_its_columns_up_to_64_rows() -> None:
+    for m in (9, 16, 17, 32, 33, 48, 49, 56, 63, 64):
+        cfg = ops._gpu_config(DEV, m, 37888, 3584, 128)
+        assert (cfg.block_n, cfg.waves_k, cfg.split_k) == (160, 4, 1), f"m={m}"
+        assert cfg.block_m == 16 * -(-m // 16), f"m={m}"

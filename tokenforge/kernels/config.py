@@ -543,11 +543,10 @@ def _model_rows(m: int) -> int:
 RETUNE_MARGIN = 0.93
 """A shipped K-split tile gives way to the modelled best at this M where the model puts that below
 this share of the tuned tile's time: well inside a bucket the tuned columns can be the wrong ones.
-Measured on MI355X on 88 calls inside the buckets (cold weights): of the 34 that give way 26 are 2 to
-27% faster (gate_up M = 80 46.6 -> 34.5 us, qkv M = 300 25.2 -> 19.6), the eight at gate_up and down
-M = 33 .. 48 within 2.5% (gate_up M = 48 29.1 -> 29.7; 26.1 -> 25.0 with warm weights). Where M rounds up to
-the bucket's own rows the tuner has measured the very tiles and its choice stands (gate_up M = 63: the
-model would take 33.7 us for 32.4)."""
+Measured on MI355X on 88 calls inside the buckets (cold weights): of the 30 that give way 26 are 2 to
+27% faster (gate_up M = 80 46.6 -> 34.5 us, qkv M = 300 25.2 -> 19.6), the four at down M = 33 .. 48
+within 1%. Where M rounds up to the bucket's own rows the tuner has measured the very tiles and its
+choice stands."""
 
 
 @functools.lru_cache(maxsize=4096)
