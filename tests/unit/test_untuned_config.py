@@ -95,6 +95,7 @@ def test_tuned_choices_fit_their_layer() -> None:
     (4096, 1024, 3, (16, 4)), (4096, 2048, 3, (16, 8)), (4096, 2944, 3, "base"), (5120, 11008, 2, "base"),
     (8192, 8192, 4, "base"), (4608, 4096, 1, "base"), (528, 4096, 3, (16, 8)), (3584, 18944, 3, (16, 16)),
     (4608, 18944, 3, "base"), (6160, 8192, 3, (16, 8)), (16400, 4096, 3, "base"), (17712, 256, 6, (16, 2)),
+    (31200, 1408, 17, "base"), (6144, 13696, 11, "base"), (31824, 256, 16, "base"),
 ])
 def test_decode_rows_keep_the_default_where_it_is_faster(n: int, k: int, m: int, kernel: object) -> None:
     cfg = untuned_config(m, n, k, 128)

@@ -456,14 +456,17 @@ def ksplit_rows(cfg: GemmConfig, m: int) -> GemmConfig:
     return replace(cfg, block_m=min(rows)) if rows else cfg
 
 
-# Time model of the two GEMM forms an untuned layer can run on, fitted (least squares over log
-# time) to 3500 launches on MI355X: ten layer shapes from 1152 x 896 to 37888 x 3584, M = 16 .. 2048,
-# every tile and split of both. Microseconds and bytes:
+# Time model of the GEMM forms an untuned layer can run on, in microseconds and bytes:
 #   T = launch + (work^q + hbm^q + l2^q)^(1/q) [+ split], work = rounds over the CUs x time of one
 # workgroup; hbm the layer, x and y once; l2 every workgroup's weights and x. A K-split workgroup runs
-# iterations of MFMAs (MT RT), dequantization (RT) and x (MT WK); a producer/consumer one K blocks of
-# 64 at its tile's rate. The config it picks is 3.4% slower than the best one in the mean over the
-# fitted shapes (at most 29%); the fixed tiles chosen by bucket before were 1.3 to 2.8 times slower.
+# iterations of MFMAs (MT RT), dequantization (RT) and x (MT WK); an LDS-tile one K blocks of 64 and a
+# skinny one K steps of 128 at its tile's rate. Fitted (least squares over log time) to launches of every
+# tile and split on ten layer shapes from 1152 x 896 to 37888 x 3584, M = 16 .. 2048, on MI355X; the two
+# tiles that were the defaults before were added beside it. bench_probes/launch_choice.py checks the
+# choice against those defaults and gives the data of a refit. Over 11481 calls on 1488 random layers
+# (M = 1 .. 8000, cold weights) it takes 0.44 to 0.89 of the default's time in the mean of a range of M;
+# 71 calls are more than 3% slower, at most 1.18 times. The modelled time is 0.88 (M > 4096) to 1.0 of
+# the measured one, with a spread of 9 to 16%.
 _NUM = {
     "launch": 1.73, "q": 1.66, "hbm": 7.57e6, "split": 2.26, "partials": 8.74e6,
     "ks_wg": 2.49, "mfma": 0.0836, "dequant": 0.172, "x": 0.0065, "pair": 1.27, "ks_l2": 25.6e6,
@@ -472,43 +475,55 @@ _NUM = {
     "pc": {(256, 192): 0.917, (256, 160): 0.803, (256, 128): 0.512, (128, 256): 0.658, (128, 128): 0.192},
     # the shared-role 256 x 256 tile, fitted to 880 launches above M = 256 beside the others' model
     "wide_wg": 7.0, "wide_block": 1.52,
+    # the default of 9 .. 32 rows (16 or 32 x 64, no LDS sums), fitted to 1640 launches the same way
+    "skinny_wg": 2.0, "skinny_step": 0.35, "skinny_l2": 50e6,
 }
 
 
+@dataclass(frozen=True)
+class _Cost:
+    """A tile's constants in the time model."""
+
+    wg_us: float  # prologue and end of a workgroup
+    iter_us: float  # an iteration (K split), a block of 64 or a step of 128 K
+    l2_rate: float  # bytes of its loads per us
+    per_cu: int = 1  # workgroups a CU holds ...
+    share: float = 1.0  # ... and the time of a round of them beside one workgroup's
+
+
 @functools.lru_cache(maxsize=None)
-def _model_tiles(group_size: int, ksplit: bool) -> tuple[tuple[GemmConfig, float, float, float, bool], ...]:
-    """(config, prologue of a workgroup, time of an iteration or block, rate of its loads, whether two
-    workgroups share a CU) of the model's candidates."""
+def _model_tiles(group_size: int, ksplit: bool) -> tuple[tuple[GemmConfig, _Cost], ...]:
+    """The model's candidate tiles (split_k 1) and their constants."""
     out = []
     for mt, rt, wk in KSPLIT_TILES if ksplit else ():
         per_iter = _NUM["mfma"] * mt * rt + _NUM["dequant"] * rt + _NUM["x"] * mt * wk
         pair = mt * rt <= 4 and rt <= 2 and mt * wk <= 8  # registers and LDS of a second workgroup
-        out.append((ksplit_config(mt, rt, wk), _NUM["ks_wg"], per_iter, _NUM["ks_l2"], pair))
+        cost = _Cost(_NUM["ks_wg"], per_iter, _NUM["ks_l2"], 2 if pair else 1, _NUM["pair"] if pair else 1.0)
+        out.append((ksplit_config(mt, rt, wk), cost))
     if group_size >= 64:
         for (bm, bn), tile in _NUM["pc"].items():
             w = 4 if (bm, bn) == (128, 128) else 8
-            out.append((GemmConfig("gemm_mfma", bm, bn, 64, 1, w, 8), _NUM["pc_wg"], _NUM["pc_block"] + tile,
-                        _NUM["pc_l2"], False))
+            out.append((GemmConfig("gemm_mfma", bm, bn, 64, 1, w, 8),
+                        _Cost(_NUM["pc_wg"], _NUM["pc_block"] + tile, _NUM["pc_l2"])))
         # Slower per column than the producer/consumer tiles but wider than any of them: the fewest
         # rounds where its tiles fill one or two (4096 x 4096 M = 3584 124 us, 256 x 128 133).
-        out.append((GemmConfig("gemm_mfma", 256, 256, 64, 1, 8, 3), _NUM["wide_wg"], _NUM["wide_block"], _NUM["pc_l2"],
-                    False))
+        out.append((GemmConfig("gemm_mfma", 256, 256, 64, 1, 8, 3),
+                    _Cost(_NUM["wide_wg"], _NUM["wide_block"], _NUM["pc_l2"])))
     return tuple(out)
 
 
-def _model_us(cfg: GemmConfig, costs: tuple[float, float, float, bool], m: int, n: int, k: int) -> float:
-    """Modelled time of ``cfg`` (a row of :func:`_model_tiles` with a split)."""
-    wg_us, iter_us, l2_rate, pair = costs
+def _model_us(cfg: GemmConfig, cost: _Cost, m: int, n: int, k: int) -> float:
+    """Modelled time of ``cfg`` (a tile with a split)."""
     q, split = _NUM["q"], cfg.split_k
     wgs = -(-m // cfg.block_m) * -(-n // cfg.block_n) * split
-    if pair and wgs > NUM_CUS:
-        rounds = -(-wgs // (2 * NUM_CUS)) * _NUM["pair"]
+    if wgs <= NUM_CUS:
+        rounds = 1.0
     else:
-        rounds = -(-wgs // NUM_CUS)
+        rounds = -(-wgs // (cost.per_cu * NUM_CUS)) * cost.share
     steps = -(-(k // 128) // split)
-    iters = -(-steps // cfg.waves_k) if cfg.ksplit else 2 * steps  # K-split iterations, blocks of 64
-    work = rounds * (wg_us + iters * iter_us)
-    l2 = wgs * (cfg.block_n * 0.53 + cfg.block_m * 2) * (k / split) / l2_rate
+    iters = -(-steps // cfg.waves_k) if cfg.ksplit else steps if cfg.skinny else 2 * steps
+    work = rounds * (cost.wg_us + iters * cost.iter_us)
+    l2 = wgs * (cfg.block_n * 0.53 + cfg.block_m * 2) * (k / split) / cost.l2_rate
     hbm = (n * k * 0.53 + m * k * 2 + m * n * 2) / _NUM["hbm"]
     us = _NUM["launch"] + (work**q + hbm**q + l2**q) ** (1 / q)
     return us + (_NUM["split"] + split * m * n * 8 / _NUM["partials"] if split > 1 else 0.0)
@@ -519,7 +534,7 @@ def _modelled_config(m: int, n: int, k: int, group_size: int) -> tuple[float, Ge
     """The modelled time and config of the fastest tile and split (None: no form serves the layer)."""
     best: tuple[float, GemmConfig] | None = None
     steps = k // 128
-    for cfg, *costs in _model_tiles(group_size, ksplit_applies(n, k)):
+    for cfg, cost in _model_tiles(group_size, ksplit_applies(n, k)):
         if cfg.ksplit and (m <= cfg.block_m - 16 or (-(-m // cfg.block_m) > 4 if m <= 128 else
                                                      cfg.block_m < 48 or cfg.block_n < 64)):
             continue  # a smaller tile holds M, or outside the fit: many small tiles refetch the weights
@@ -528,7 +543,7 @@ def _modelled_config(m: int, n: int, k: int, group_size: int) -> tuple[float, Ge
             if split > 1 and (tiles * split > 2 * NUM_CUS or steps < split * (cfg.waves_k if cfg.ksplit else 2)):
                 break
             split_cfg = replace(cfg, split_k=split)
-            us = _model_us(split_cfg, tuple(costs), m, n, k)
+            us = _model_us(split_cfg, cost, m, n, k)
             if best is None or us < best[0]:
                 best = (us, split_cfg)
     return best
@@ -552,10 +567,10 @@ choice stands."""
 @functools.lru_cache(maxsize=4096)
 def _retiled(cfg: GemmConfig, m: int, n: int, k: int, group_size: int) -> GemmConfig:
     best = _modelled_config(m, n, k, group_size)
-    tiles = {c.variant(): costs for c, *costs in _model_tiles(group_size, True)}
+    tiles = {c.variant(): cost for c, cost in _model_tiles(group_size, True)}
     if best is None or cfg.variant() not in tiles:
         return cfg
-    tuned = _model_us(cfg, tuple(tiles[cfg.variant()]), m, n, k)
+    tuned = _model_us(cfg, tiles[cfg.variant()], m, n, k)
     return best[1] if best[0] < RETUNE_MARGIN * tuned else cfg
 
 
@@ -605,7 +620,9 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     * M <= 4 below that: :func:`_narrow_decode_config`.
     * M = 5 .. 8: a wide layer of few weights as at M <= 4 (K too short for the stream form: 17712 x 256
       4.4 us against 5.7 for the tile), the others the modelled tile (512 x 4096 5.6 us against 8.2).
-    * M > 8: the modelled best of the K-split, the producer/consumer and the 256 x 256 tiles.
+    * M > 8: the modelled best of the K-split, the producer/consumer and the 256 x 256 tiles; up to M = 32
+      the bucket's default where the model puts that first (its tiles come three or two to a CU: 31200 x
+      1408 M = 17 10.7 us against 11.9, 6144 x 13696 M = 11 17.0 against 18.8).
     """
     bucket = MAX_BUCKET_M if m > MAX_BUCKET_M else m_bucket(m)
     base = default_config(bucket, n, k, group_size)
@@ -621,7 +638,13 @@ def untuned_config(m: int, n: int, k: int, group_size: int, x_bytes: int = 0) ->
     if m <= STREAM_MAX_M or (m <= STREAM_WIDE_M and n >= 640 * 16 and n * k <= 12 << 20):
         return _narrow_decode_config(m, n, k, base)
     best = _modelled_config(_model_rows(m), n, k, group_size)
-    return base if best is None else best[1]
+    if best is None:
+        return base
+    if STREAM_WIDE_M < m <= 32:
+        skinny = _Cost(_NUM["skinny_wg"], _NUM["skinny_step"], _NUM["skinny_l2"], 3 if base.block_m == 16 else 2)
+        if _model_us(base, skinny, m, n, k) < best[0]:
+            return base
+    return best[1]
 
 
 def candidate_configs(bucket: int, group_size: int) -> list[GemmConfig]:
