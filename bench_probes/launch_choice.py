@@ -3,9 +3,9 @@ picks beside the bucket's default, and its modelled time beside the measured one
 
 Usage (needs the GPU)::
 
-    python bench_probes/launch_choice.py time SEED SECONDS > gpurun_out/launch_choice.log
-    python bench_probes/launch_choice.py tiles N K GROUP M [M ...] >> gpurun_out/launch_choice.log
-    python bench_probes/launch_choice.py summary gpurun_out/launch_choice.log   # profiles/untuned_launch_choice.md
+    python bench_probes/launch_choice.py time SEED SECONDS > launch_choice.log
+    python bench_probes/launch_choice.py tiles N K GROUP M [M ...] >> launch_choice.log
+    python bench_probes/launch_choice.py summary launch_choice.log   # profiles/untuned_launch_choice.md
 
 ``time`` draws layers (N 256 .. 32768 in steps of 8, K 256 .. 16384 in steps of 128, groups of 32, 64 and
 128) and eight M from 1 to 8000 each, until SECONDS have passed. ``tiles`` times every tile and K split of
@@ -130,8 +130,8 @@ def summary(log: str) -> None:
         "",
         "```",
         "R=<repo root>",
-        "python $R/bench_probes/launch_choice.py time SEED SECONDS > $R/gpurun_out/launch_choice.log",
-        "python $R/bench_probes/launch_choice.py summary $R/gpurun_out/launch_choice.log",
+        "python $R/bench_probes/launch_choice.py time SEED SECONDS > launch_choice.log",
+        "python $R/bench_probes/launch_choice.py summary launch_choice.log",
         "```",
         "",
         f"{len(rows)} calls on {len({(r['n'], r['k'], r['group']) for r in rows})} random layers, cold weights,",

@@ -114,7 +114,8 @@ int tf_w4a16_dequant(const int32_t* qweight_t, const uint16_t* scales,
 /* Kernel families (the `kernel` field of tf_gemm_config). */
 #define TF_KERNEL_GEMV_DOT 0   /* decode: in-register dequant + VALU dot2, M <= 4     */
 #define TF_KERNEL_GEMV_MFMA 1  /* decode: in-register dequant + fp16 MFMA (M <= 32)   */
-#define TF_KERNEL_GEMM_MFMA 2  /* prefill: LDS-staged dequant + fp16 MFMA, split-K    */
+#define TF_KERNEL_GEMM_MFMA 2  /* M >= 5: fp16 MFMA, weights dequantized through LDS or (block_k
+                                  128) straight into the MFMA operand, split-K              */
 #define TF_KERNEL_GEMM_FP8 3   /* W4A8 prefill (tf_w4a8_linear_ex only): e4m3 x and exact
                                   e4m3 (q - z) on the fp8 MFMA, group scale in fp32 after each
                                   128-K group; group_size 128, N % 16 == 0, split-K           */
@@ -170,8 +171,8 @@ int tf_w4a16_linear(const uint16_t* x, int64_t ldx, const int32_t* qweight_t,
 #define TF_EPILOGUE_RESIDUAL 1
 #define TF_EPILOGUE_SILU_MUL 2
 
-/* Workspace bytes of tf_w4a16_linear_ex (the LDS-tile GEMMs reduce a SiLU*mul epilogue
- * through fp32 partials even without split-K). */
+/* Workspace bytes of tf_w4a16_linear_ex (the fp32 partials of a K split; the two-buffer GEMM,
+ * num_stages 2, stages fp16 y rows for a SiLU*mul epilogue without one). */
 int64_t tf_w4a16_workspace_bytes_ex(int64_t m, int64_t n, int64_t k, int32_t group_size,
                                     const tf_gemm_config* cfg, int32_t epilogue);
 
@@ -187,7 +188,7 @@ int tf_w4a16_linear_ex(const uint16_t* x, int64_t ldx, const int32_t* qweight_t,
 /* tf_w4a16_linear_ex that allocates nothing. No counterpart in the reference: for callers that
  * cannot allocate device memory (code under HIP-graph capture that must not call hipMalloc,
  * tight serving loops, harnesses that forbid allocation). The workspace the kernels need
- * (split-K partials, the SiLU*mul rows of the LDS-tile GEMMs) comes from a fixed device array
+ * (split-K partials, the SiLU*mul rows of the two-buffer GEMM) comes from a fixed device array
  * of tf_noalloc_scratch_bytes() bytes (32 MiB) that each GPU holds until the process ends; a
  * call needing more is rejected (TF_EINVAL). Nothing needs clearing between calls. All calls
  * on one GPU share that array: calls that overlap in time on one GPU (other streams, other
@@ -207,8 +208,8 @@ int tf_w4a16_linear_ex_noalloc(const uint16_t* x, int64_t ldx, const int32_t* qw
  * xscale fp32, row m at xscale[m * xscale_stride] (stride 0: one scale for every row).
  * e4m3 values are exact in fp16, so with xscale = 1 this equals tf_w4a16_linear on the
  * decoded x bit for bit. Epilogues as tf_w4a16_linear_ex (applied after the row scale).
- * The GEMV configs decode the codes while staging x in LDS; the GEMM configs decode x to fp16
- * into the workspace first. Every check runs before anything is launched. */
+ * The GEMV configs decode the codes while staging x in LDS; the gemm_mfma configs decode x to
+ * fp16 into the workspace first; gemm_fp8 multiplies the codes. Every check runs before anything is launched. */
 int64_t tf_w4a8_workspace_bytes_ex(int64_t m, int64_t n, int64_t k, int32_t group_size,
                                    const tf_gemm_config* cfg, int32_t epilogue);
 int tf_w4a8_linear_ex(const uint8_t* x8, int64_t ldx8, const float* xscale, int64_t xscale_stride,

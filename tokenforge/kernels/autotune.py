@@ -1,12 +1,12 @@
 """Persistent autotune cache for the gfx950 W4A16 kernels (autotune.py:1-267 in the reference).
 
 Tuning runs eagerly at weight-load time (``process_weights_after_loading``), before HIP
-graphs are captured. The hot path only does a dict lookup and falls back to the heuristic
-:func:`config.default_config` on a miss, so a call never benchmarks, allocates for tuning, or
-synchronizes.
+graphs are captured. The hot path only does a dict lookup; on a miss the operators take
+:func:`config.untuned_config` (and :func:`lookup` itself the bucket's heuristic
+:func:`config.default_config`), so a call never benchmarks, allocates for tuning, or synchronizes.
 
 Lookups fall back to a table shipped in ``tokenforge/kernels/tuned/`` (same format, tuned on
-MI355X for the Qwen2.5-7B decoder shapes) and then to the heuristic default.
+MI355X for the Qwen2.5-7B decoder shapes) before that.
 
 The cache lives at ``$TOKENFORGE_CACHE_DIR`` (default ``~/.cache/tokenforge``) as
 ``<gpu>-hip<abi>.json``: ``<gpu>`` is ``device.gpu_identity`` (e.g. ``amd-gfx950-256cu``)

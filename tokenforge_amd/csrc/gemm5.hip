@@ -15,11 +15,11 @@
 // times the bytes of the weights in x, and read 1 KB of LDS per MFMA). Splitting K over the waves
 // instead of the columns lets BN be chosen for the grid (a whole round of tiles over the CUs) with
 // eight waves in flight in any case, and needs no second kernel, unlike a K split over workgroups.
-// Measured on MI355X against the fastest of the other forms (us): gate_up (37888 x 3584) M = 16
-// 17.6 / 20.1, M = 48 23.5 / 31.5 (the layer's bytes alone take 14); 4608 x 3584 M = 100 11.5 / 15.8,
-// M = 512 24.5 / 33.2; 896 x 4864 M = 100 7.2 / 9.5; 3584 x 18944 M = 64 19.9 / 23.1. Past M = 128 the
-// LDS-tile GEMMs, which dequantize a weight once per 256 rows, take over as soon as their tiles
-// fill the CUs.
+// Measured on MI355X against the fastest of the other forms (us, cold weights): gate_up (37888 x 3584)
+// with SiLU*mul M = 16 23.3 / 26.8, M = 32 26.4 / 32.1, M = 64 32.7 / 46.9 (a pure read of the layer's
+// loads takes 14.7); 3584 x 3584 M = 16 6.6 / 8.2; 4608 x 3584 M = 128 13.5 / 19.3, M = 512 27.9 / 36.7;
+// 3584 x 18944 M = 64 22.8 / 27.2. Past M = 128 the LDS-tile GEMMs, which dequantize a weight once per 256
+// rows, take over as soon as their tiles fill the CUs.
 //
 // LDS rows hold 16 chunks of 16 bytes (one 256-byte bank line); chunk c of row r sits in slot
 // c ^ (r & 11), free of bank conflicts for the fragment reads (lane 16 g + c at row c, chunk

@@ -1,7 +1,7 @@
 // tf_w4a16_linear_ex_noalloc: tf_w4a16_linear_ex for callers that cannot allocate.
 //
-// The kernels that need a workspace (split-K partials of the GEMMs, the fp32 rows the LDS-tile
-// GEMMs reduce a SiLU*mul epilogue through) get it from `scratch`, a fixed device array of
+// The kernels that need a workspace (split-K partials, the fp16 rows the two-buffer GEMM stages
+// for a SiLU*mul epilogue) get it from `scratch`, a fixed device array of
 // kScratchBytes that every GPU the library runs on holds until the process ends. Nothing here
 // calls hipMalloc, hipFree or any allocating routine. The array's device address is looked up
 // once per device (hipGetSymbolAddress, with that device current) on the entry point's first
