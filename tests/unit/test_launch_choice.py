@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from tokenforge.kernels import _lib, autotune, ops
-from tokenforge.kernels.config import fill_split, ksplit_config, ksplit_rows
+from tokenforge.kernels.config import SPAN_32BIT, default_config, fill_split, ksplit_config, ksplit_rows
 from tokenforge.kernels.metrics import KERNEL_CALLS
 
 FAMILY_OF = {_lib.KERNEL_IDS[k]: ("hip_gemm" if k in ("gemm_mfma", "gemm_fp8") else "hip_gemv") for k in _lib.KERNEL_IDS}
@@ -77,3 +77,10 @@ def test_gate_up_keeps_its_columns_up_to_64_rows() -> None:
         cfg = ops._gpu_config(DEV, m, 37888, 3584, 128)
         assert (cfg.block_n, cfg.waves_k, cfg.split_k) == (160, 4, 1), f"m={m}"
         assert cfg.block_m == 16 * -(-m // 16), f"m={m}"
+
+
+def test_rows_past_32_bit_offsets_leave_a_tuned_tile() -> None:
+    n, k, g = 1024, 1024, 32
+    autotune.get_cache("amd-gfx950-256cu").put(256, n, k, g, ksplit_config(3, 4, 4))
+    assert ops._gpu_config(DEV, 200, n, k, g, SPAN_32BIT - 2).ksplit
+    assert ops._gpu_config(DEV, 200, n, k, g, SPAN_32BIT) == default_config(256, n, k, g)

@@ -64,7 +64,9 @@ from tokenforge.kernels.config import (
     M_BUCKETS,
     MAX_BUCKET_M,
     NUM_CUS,
+    SPAN_32BIT,
     GemmConfig,
+    default_config,
     fp8_gemm_applies,
     fp8_gemm_config,
     norm_fused_config,
@@ -133,6 +135,8 @@ def _gpu_config(device: torch.device, m: int, n: int, k: int, group_size: int, x
         cfg = untuned_config(m, n, k, group_size, x_bytes)
     else:
         cfg = tuned_at(autotune.lookup(*key), m, n, k, group_size, own=source == "cache")
+        if cfg.ksplit and x_bytes >= SPAN_32BIT:  # as an untuned layer's: past the tile's offsets
+            cfg = default_config(key[1], n, k, group_size)
     if m > MAX_BUCKET_M and cfg.split_k > 1 and -(-m // cfg.block_m) * -(-n // cfg.block_n) >= NUM_CUS:
         # Above the largest bucket its config is reused; once the M tiles alone fill the CUs a
         # K split only adds the fp32 workspace (split * M * N * 4 bytes) and its reduction.
