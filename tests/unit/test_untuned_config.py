@@ -93,6 +93,7 @@ def test_tuned_choices_fit_their_layer() -> None:
 
 @pytest.mark.parametrize(("n", "k", "m", "kernel"), [
     (4096, 1024, 3, (16, 4)), (4096, 2048, 3, (16, 8)), (4096, 2944, 3, "base"), (5120, 11008, 2, "base"),
+    (4096, 2048, 2, (16, 4)), (8192, 4096, 2, (16, 8)), (4096, 11008, 4, (16, 16)), (4096, 5632, 2, (16, 16)),
     (8192, 8192, 4, "base"), (4608, 4096, 1, "base"), (528, 4096, 3, (16, 8)), (3584, 18944, 3, (16, 16)),
     (4608, 18944, 3, "base"), (6160, 8192, 3, (16, 8)), (16400, 4096, 3, "base"), (17712, 256, 6, (16, 2)),
     (31200, 1408, 17, "base"), (6144, 13696, 11, "base"), (31824, 256, 16, "base"),

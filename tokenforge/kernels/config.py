@@ -463,10 +463,10 @@ def ksplit_rows(cfg: GemmConfig, m: int) -> GemmConfig:
 # skinny one K steps of 128 at its tile's rate. Fitted (least squares over log time) to launches of every
 # tile and split on ten layer shapes from 1152 x 896 to 37888 x 3584, M = 16 .. 2048, on MI355X; the two
 # tiles that were the defaults before were added beside it. bench_probes/launch_choice.py checks the
-# choice against those defaults and gives the data of a refit. Over 11481 calls on 1488 random layers
-# (M = 1 .. 8000, cold weights) it takes 0.44 to 0.89 of the default's time in the mean of a range of M;
-# 71 calls are more than 3% slower, at most 1.18 times. The modelled time is 0.88 (M > 4096) to 1.0 of
-# the measured one, with a spread of 9 to 16%.
+# choice against those defaults and gives the data of a refit. Over 10986 calls on random layers (M = 1
+# .. 8000, cold weights) it takes 0.46 to 0.89 of the default's time in the mean of a range of M; 78 calls
+# are more than 3% slower, at most 1.28 times. The modelled time is 0.84 (M > 4096) to 1.0 of the measured
+# one, with a spread of 9 to 16%.
 _NUM = {
     "launch": 1.73, "q": 1.66, "hbm": 7.57e6, "split": 2.26, "partials": 8.74e6,
     "ks_wg": 2.49, "mfma": 0.0836, "dequant": 0.172, "x": 0.0065, "pair": 1.27, "ks_l2": 25.6e6,
@@ -590,21 +590,33 @@ def _narrow_decode_config(m: int, n: int, k: int, base: GemmConfig) -> GemmConfi
     """The M <= 4 choice between ``base``, the bucket's default (the stream form, or the 32-column GEMV
     where that does not run), and the GEMV with 16 columns a workgroup.
 
-    Against the stream form at M = 1 base; at M = 2 .. 4 the GEMV up to K = 2048, with 4 waves up to K =
-    1024 and 8 above (M = 3, GEMV / stream: 2048 x 1024 4.0 / 4.3 us, 4608 x 2048 5.3 / 6.1; longer K
-    4096 x 2944 6.1 / 5.4, 5120 x 11008 15.2 / 13.7, 4608 x 4096 8.1 / 7.4). Against the 32-column GEMV:
-    while its workgroups are one round over the CUs (N <= 4096) always, with 4, 8 or 16 waves by K (528
-    x 4096, M = 3 5.3 / 7.0; 3584 x 18944 11.7 / 17.8); past that 4 waves below K = 4096 and 64M
-    weights and 8 up to K = 8192 (6160 x 8192 11.6 / 12.3; 4608 x 18944 24.5 / 20.9, 16400 x 4096 14.8 /
-    14.4, 20432 x 3840 at M = 4 18.8 / 16.5). Over 800 calls of 1 to 8 rows on 140 random layers the choice
-    took 0.78 of the default's time in the mean, at most 1.04."""
+    Against the stream form, which stages every row of x whole: at M = 1 base; at M = 2 the GEMV up to K =
+    4096, with 4 waves up to K = 2048 and 8 above, at M = 3 up to K = 2432 and at M = 4 up to K = 2048, with
+    4 waves up to K = 1024 and 8 above; and with 16 waves for longer K (from K = 7168 at M = 3 and 4) while
+    its workgroups are one round over the CUs (N <= 4096). GEMV / stream in us, cold weights; weights in the Infinity
+    Cache: M = 2 4608 x 4096 7.0 / 7.3; 6.1 / 7.0, 2048 x 8192 7.0 / 7.7; 6.1 / 6.6, M = 3 2048 x 1024 4.0 /
+    4.3; 3.6 / 4.1, 4608 x 2048 5.3 / 6.1; 5.0 / 5.8, 2048 x 8192 8.0 / 8.1; 6.7 / 7.1. On the other side M
+    = 2 5120 x 5632 9.2 / 8.6; 7.4 / 7.9 (8 waves), M = 3 2048 x 5632 6.7 / 6.2; 6.2 / 5.9, 5120 x 11008 15.2
+    / 13.7; 11.8 / 11.4, 4608 x 4096 8.1 / 7.4; 6.5 / 7.0 (a model of such layers does not fit the cache).
+    Against the 32-column GEMV: while it is one round always, with 4, 8 or 16 waves by K (528 x 4096, M =
+    3 5.3 / 7.0; 3584 x 18944 in groups of 32 14.4 / 20.6); past that 4 waves below K = 4096 and 64M
+    weights and 8 up to K = 8192, or any K where the 32-column grid is past one round too (6160 x 8192
+    11.6 / 12.3, 8208 x 11008 23.4 / 29.2; 4608 x 18944 24.5 / 20.9, 16400 x 4096 14.8 / 14.4, 20432 x 3840
+    at M = 4 18.8 / 16.5)."""
     steps = k // 128
-    if base.stream:
-        waves = 0 if m == 1 or steps > 16 else 4 if steps <= 8 else 8
-    elif n <= 16 * NUM_CUS:
+    one_round = n <= 16 * NUM_CUS
+    if base.stream and m == 1:
+        waves = 0
+    elif base.stream and m == 2:
+        waves = 4 if steps <= 16 else 8 if steps <= 32 else 16 if one_round else 0
+    elif base.stream:
+        waves = 4 if steps <= 8 else 8 if steps <= (19 if m == 3 else 16) else 16 if one_round and steps >= 56 else 0
+    elif one_round:
         waves = 4 if steps < 32 else 8 if steps < 56 else 16
+    elif steps < 32:
+        waves = 4 if n * k <= 64 << 20 else 0
     else:
-        waves = (4 if n * k <= 64 << 20 else 0) if steps < 32 else 8 if steps <= 64 and n < 640 * 16 else 0
+        waves = 8 if n < 640 * 16 and (steps <= 64 or n > 32 * NUM_CUS) else 0
     return GemmConfig("gemv_mfma", 16, 16, 128, 1, min(waves, _pow2_at_most(steps, 16)), 2) if waves else base
 
 
