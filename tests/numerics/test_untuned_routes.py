@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize(("n", "k", "g", "ms"), [
     (512, 1024, 128, SMALL_M), (512, 1152, 64, SMALL_M), (512, 2176, 32, SMALL_M), (520, 1024, 64, SMALL_M),
-    (4096, 512, 128, SMALL_M), (4112, 4224, 128, SMALL_M), (4112, 8320, 64, SMALL_M), (10240, 384, 128, SMALL_M),
+    (512, 7296, 64, SMALL_M), (8224, 4224, 128, SMALL_M), (8208, 8320, 128, SMALL_M), (4096, 512, 128, SMALL_M), (4112, 4224, 128, SMALL_M), (4112, 8320, 64, SMALL_M), (10240, 384, 128, SMALL_M),
     (10256, 1280, 32, SMALL_M), (10240, 4096, 128, SMALL_M), (256, 12544, 128, SMALL_M), (3600, 640, 128, (129, 1025)),
     (264, 320, 64, (129, 300, 1025)), (272, 384, 32, (129, 1025)), (3848, 256, 64, (3585,)),
 ])
