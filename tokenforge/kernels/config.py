@@ -463,9 +463,9 @@ def ksplit_rows(cfg: GemmConfig, m: int) -> GemmConfig:
 # skinny one K steps of 128 at its tile's rate. Fitted (least squares over log time) to launches of every
 # tile and split on ten layer shapes from 1152 x 896 to 37888 x 3584, M = 16 .. 2048, on MI355X; the two
 # tiles that were the defaults before were added beside it. bench_probes/launch_choice.py checks the
-# choice against those defaults and gives the data of a refit. Over 10986 calls on random layers (M = 1
-# .. 8000, cold weights) it takes 0.46 to 0.89 of the default's time in the mean of a range of M; 78 calls
-# are more than 3% slower, at most 1.28 times. The modelled time is 0.84 (M > 4096) to 1.0 of the measured
+# choice against those defaults and gives the data of a refit. Over 11295 calls on 1465 random layers (M
+# = 1 .. 8000, cold weights) it takes 0.45 to 0.88 of the default's time in the mean of a range of M; 69
+# calls are more than 3% slower, at most 1.25 times. The modelled time is 0.84 (M > 4096) to 1.0 of the measured
 # one, with a spread of 9 to 16%.
 _NUM = {
     "launch": 1.73, "q": 1.66, "hbm": 7.57e6, "split": 2.26, "partials": 8.74e6,
